@@ -100,6 +100,8 @@ SIGNATURES = {
     "haste_rewire": (ctypes.c_int, [_P, _I32, _P, _P, _P, _I64, _I64, _I64, _I64, _I32, _F32,
                                     _I64, _I32, _I32, _F32, _U64, _P]),
     "haste_rewire_scores": (ctypes.c_int, [_P, _I32, _P, _I32, _I32, _P, _I64, _I64, _I64, _P]),
+    "haste_rewire_select_workspace_size": (_I64, []),
+    "haste_rewire_select": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _I64, _P]),
     "haste_rewire_ex": (ctypes.c_int, [_P, _I32, _P, _P, _I32, _I32, _P, _P, _P, _P, _I64, _I64,
                                        _I64, _I64, _I32, _F32, _I64, _I32, _I32, _F32, _U64,
                                        _P]),

@@ -226,6 +226,12 @@ __device__ __forceinline__ int slot_rank(const float* sc, int* part, int F, int 
     return rank;
 }
 
+// Key of a slot (numbered over the layer) in the order of GLOBAL_FRACTION: by the
+// bits of its score, then by slot.  Scores are >= 0, whose bits order them.
+__device__ __forceinline__ int64_t slot_key(float score, int64_t slot) {
+    return ((int64_t)__float_as_uint(score) << 32) | (int64_t)(uint32_t)slot;
+}
+
 // A 16-byte piece holding W[l, c .. c + 16/es - 1] with its pruned elements
 // (bit e of bits: element c + e) set to their new values.
 template <int WD>
@@ -307,8 +313,12 @@ __device__ __forceinline__ void load_pieces(u32x4 (&v)[NPT], rsrc_t rs, int tid)
 }
 
 // Whole groups: every group's rows fit one LDS stage (NPT pieces of 16 bytes
-// per thread) and start and end on 16-byte boundaries, no gradient, scores
-// computed here.  A persistent grid: workgroup b takes groups b, b + gridDim.x,
+// per thread) and start and end on 16-byte boundaries.  GIVEN: the layer's
+// scores are scores_in (and key_thr the last pruned key of GLOBAL_FRACTION);
+// otherwise they are computed here, without a gradient.  Bound by HBM: W is read
+// and written once (and by the Philox draws of RANDOM initial weights).  A given
+// score set took rewire_kernel's column stores before, 2 bytes per row of a
+// pruned slot: 41 us at 131,073 labels (G = 64, F = 128, RANDOM), 33 here.  A persistent grid: workgroup b takes groups b, b + gridDim.x,
 // ...; the next group's rows and indices are loaded into registers while the
 // current group is scored from LDS; a group with pruned slots goes back whole
 // with 16-byte stores; one atomic per workgroup adds its pruned count.  Pruned
@@ -316,12 +326,12 @@ __device__ __forceinline__ void load_pieces(u32x4 (&v)[NPT], rsrc_t rs, int tid)
 // (rewire_regrow_kernel).  All global accesses go through buffer
 // resources with out-of-range offsets for the ones a lane skips, so that the
 // loads of the next group are waited for by count.
-template <int WD, int NPT>
+template <int WD, int NPT, bool GIVEN>
 __global__ __launch_bounds__(kThreads, 4) void rewire_whole_kernel(
     void* __restrict__ W, int32_t* __restrict__ idx, float* __restrict__ scores_out,
     int32_t* __restrict__ n_pruned, int64_t O, int F, int G, int D, int prune_mode, float thr,
     int k, int regrow_mode, int init_mode, float bound, uint32_t k0, uint32_t k1, int score_mode,
-    int64_t Gc) {
+    const float* __restrict__ scores_in, const int64_t* __restrict__ key_thr, int64_t Gc) {
     using Wt = El<WD>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float* sc = reinterpret_cast<float*>(smem);
@@ -348,6 +358,12 @@ __global__ __launch_bounds__(kThreads, 4) void rewire_whole_kernel(
     int64_t g = blockIdx.x;
     u32x4 v[NPT];
     load_pieces(v, w_rsrc(g), tid);
+    // GIVEN: the group's scores, and the key of the last pruned slot
+    auto given = [&](int64_t gg) {
+        return GIVEN && jv && gg < Gc ? scores_in[gg * F + tid] : 0.0f;
+    };
+    float sgiven = given(g);
+    const int64_t kthr = GIVEN && key_thr != nullptr ? *key_thr : 0;
     for (; g < Gc; g += gridDim.x) {
         const int64_t l0 = g * G;
         const int rows = (int)min((int64_t)G, O - l0);
@@ -362,7 +378,11 @@ __global__ __launch_bounds__(kThreads, 4) void rewire_whole_kernel(
         load_pieces(v, w_rsrc(g + gridDim.x), tid);
 
         float score = 0.0f;
-        if (jv) {
+        if constexpr (GIVEN) {
+            score = sgiven;
+            sgiven = given(g + gridDim.x);
+            if (jv) sc[tid] = score;
+        } else if (jv) {
             score = mx ? column_score<WD, -1, true>(stw, nullptr, rows, F, tid, -__builtin_inff())
                        : column_score<WD, -1, false>(stw, nullptr, rows, F, tid, 0.0f) /
                              (float)rows;
@@ -375,6 +395,8 @@ __global__ __launch_bounds__(kThreads, 4) void rewire_whole_kernel(
         if (prune_mode == HASTE_PRUNE_FRACTION) {
             __syncthreads();
             m = slot_rank(sc, part, F, tid) < k && jv;
+        } else if (GIVEN && prune_mode == HASTE_PRUNE_GLOBAL_FRACTION) {
+            m = jv && slot_key(score, g * F + tid) <= kthr;
         } else {
             m = jv && score < thr;
         }
@@ -418,8 +440,8 @@ __global__ __launch_bounds__(kThreads) void rewire_scores_kernel(
     if ((int)threadIdx.x < F) scores[g * F + threadIdx.x] = s;
 }
 
-// Every other case (rows over several LDS chunks, rows off 16-byte boundaries,
-// a gradient, or the layer's scores given): a persistent grid over the groups,
+// Every other case (rows over several LDS chunks, rows off 16-byte boundaries, or
+// a gradient to score with): a persistent grid over the groups,
 // each scored in row chunks (or read from scores_in), the pruned slots' new
 // weights stored element by element down their columns, one atomic per
 // workgroup.  scores_in: the layer's scores (GLOBAL_FRACTION, written by
@@ -464,9 +486,7 @@ __global__ __launch_bounds__(kThreads) void rewire_kernel(
             __syncthreads();
             m = slot_rank(sc, part, F, j) < k && jv;
         } else if (prune_mode == HASTE_PRUNE_GLOBAL_FRACTION) {
-            const int64_t key =
-                ((int64_t)__float_as_uint(score) << 32) | (int64_t)(uint32_t)(g * F + j);
-            m = jv && key <= *key_thr;
+            m = jv && slot_key(score, g * F + j) <= *key_thr;
         } else {
             m = jv && score < thr;
         }
@@ -537,6 +557,157 @@ __global__ __launch_bounds__(kThreads) void rewire_regrow_kernel(int32_t* __rest
 #pragma unroll
     for (int s = 0; s < kSlotsPerLane; ++s)
         if (pr[s]) idx[g * F + lane + 64 * s] = cur[s];
+}
+
+// ---- the key of GLOBAL_FRACTION's last pruned slot: the k-th smallest slot_key of
+// the layer's scores, by radix selection of the score (three passes of 11, 11
+// and 10 bits), then of the slot among those of equal score.  Each pass
+// histograms the digit of the scores whose higher digits are settled; the next
+// launch's workgroups scan that histogram for the digit that holds rank k.  The
+// scores are read four times from the L2 (1 MB at 262,144 slots): the launches
+// bound it (five, 27 us at that size).  torch.kthvalue on 64-bit keys runs in one
+// workgroup: 1671 us there, and the whole rewire went from 1313 to 68 us.
+// Workspace (uint32): 3 histograms, the ties per chunk, then per pass the
+// settled digits and the rank left among the scores that share them.
+constexpr int kSelBins = 2048;
+constexpr int kSelChunks = 1024;   // the tie pass's workgroups
+constexpr int kSelThreads = 1024;  // of the last launch, one workgroup
+constexpr int kSelTies = 3 * kSelBins;
+constexpr int kSelState = kSelTies + kSelChunks;  // (digits, rank) after passes 0, 1, 2
+constexpr int kSelWords = kSelState + 8;
+
+// Score bits in the unsigned order of the signed keys.
+__device__ __forceinline__ uint32_t sel_bits(float s) { return __float_as_uint(s) ^ 0x80000000u; }
+
+// The bin of h[0 .. nbins) that holds rank k (1-based) and the rank within it,
+// by the workgroup's NT threads (nbins a multiple of NT); s: NT + 2 words of LDS.
+template <int NT>
+__device__ __forceinline__ void find_bin(const uint32_t* __restrict__ h, int nbins, uint32_t k,
+                                         uint32_t* s, uint32_t* bin, uint32_t* left) {
+    const int tid = threadIdx.x, per = nbins / NT;
+    uint32_t sum = 0;
+    for (int i = 0; i < per; ++i) sum += h[tid * per + i];
+    s[tid] = sum;
+    __syncthreads();
+    for (int d = 1; d < NT; d <<= 1) {  // inclusive scan
+        const uint32_t v = tid >= d ? s[tid - d] : 0u;
+        __syncthreads();
+        s[tid] += v;
+        __syncthreads();
+    }
+    const uint32_t before = s[tid] - sum;
+    if (before < k && k <= s[tid]) {
+        uint32_t c = before;
+        int i = 0;
+        while (c + h[tid * per + i] < k) c += h[tid * per + i++];
+        s[NT] = (uint32_t)(tid * per + i);
+        s[NT + 1] = k - c;
+    }
+    __syncthreads();
+    *bin = s[NT];
+    *left = s[NT + 1];
+}
+
+// The digits settled before pass P and the rank left: of pass P-2 from the
+// state, of pass P-1 by a scan of its histogram; workgroup 0 stores them.
+template <int P, int NT>
+__device__ __forceinline__ void sel_settle(uint32_t* ws, uint32_t k, uint32_t* s,
+                                           uint32_t* digits, uint32_t* left) {
+    uint32_t d = 0, r = k;
+    if constexpr (P >= 2) {
+        d = ws[kSelState + 2 * (P - 2)];
+        r = ws[kSelState + 2 * (P - 2) + 1];
+    }
+    if constexpr (P >= 1) {
+        uint32_t bin;
+        find_bin<NT>(ws + (P - 1) * kSelBins, kSelBins, r, s, &bin, &r);
+        d = (d << (P == 3 ? 10 : 11)) | bin;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            ws[kSelState + 2 * (P - 1)] = d;
+            ws[kSelState + 2 * (P - 1) + 1] = r;
+        }
+    }
+    *digits = d;
+    *left = r;
+}
+
+template <int P>
+__global__ __launch_bounds__(kThreads) void select_pass_kernel(const float* __restrict__ scores,
+                                                               int64_t n, uint32_t k,
+                                                               uint32_t* __restrict__ ws) {
+    __shared__ uint32_t hist[kSelBins];
+    __shared__ uint32_t s[kThreads + 2];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < kSelBins; i += kThreads) hist[i] = 0u;
+    uint32_t digits, left;
+    sel_settle<P, kThreads>(ws, k, s, &digits, &left);
+    __syncthreads();
+    const int64_t stride = (int64_t)gridDim.x * kThreads;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + tid; i - tid < n; i += stride) {
+        const uint32_t u = i < n ? sel_bits(scores[i]) : 0u;
+        const bool in = i < n && (P == 0 || u >> (P == 1 ? 21 : 10) == digits);
+        const uint32_t d = P == 0 ? u >> 21 : P == 1 ? (u >> 10) & 2047u : u & 1023u;
+        // a layer's scores share their first digits: the lanes with the first
+        // counted lane's digit go in as one addition
+        const uint64_t any = __ballot(in);
+        if (any == 0) continue;
+        const uint32_t d0 = (uint32_t)__shfl((int)d, __builtin_ctzll(any), 64);
+        const uint64_t same = __ballot(in && d == d0);
+        if ((tid & 63) == 0) atomicAdd(&hist[d0], (uint32_t)__popcll(same));
+        if (in && d != d0) atomicAdd(&hist[d], 1u);
+    }
+    __syncthreads();
+    for (int i = tid; i < kSelBins; i += kThreads)
+        if (hist[i] != 0u) atomicAdd(&ws[P * kSelBins + i], hist[i]);
+}
+
+// Scores equal to the k-th, per chunk of consecutive slots (chunk = workgroup).
+__global__ __launch_bounds__(kThreads) void select_ties_kernel(const float* __restrict__ scores,
+                                                               int64_t n, int64_t chunk,
+                                                               uint32_t k,
+                                                               uint32_t* __restrict__ ws) {
+    __shared__ uint32_t s[kThreads + 2];
+    uint32_t u, left;
+    sel_settle<3, kThreads>(ws, k, s, &u, &left);
+    const int64_t i0 = blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+    uint32_t c = 0;
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) c += sel_bits(scores[i]) == u;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) c += (uint32_t)__shfl_xor((int)c, m, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) ws[kSelTies + blockIdx.x] = s[0] + s[1] + s[2] + s[3];
+}
+
+// One workgroup: the chunk, then the slot, of the tie of the rank left.
+__global__ __launch_bounds__(kSelThreads) void select_key_kernel(const float* __restrict__ scores,
+                                                                 int64_t n, int64_t chunk,
+                                                                 const uint32_t* __restrict__ ws,
+                                                                 int64_t* __restrict__ key) {
+    __shared__ uint32_t s[kSelThreads + 2];
+    const uint32_t u = ws[kSelState + 4], left = ws[kSelState + 5];
+    uint32_t c, r;
+    find_bin<kSelThreads>(ws + kSelTies, kSelChunks, left, s, &c, &r);
+    const int64_t i0 = c * chunk, i1 = min(n, i0 + chunk);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int64_t b = i0; b < i1; b += kSelThreads) {
+        const int64_t i = b + threadIdx.x;
+        const bool tie = i < i1 && sel_bits(scores[i]) == u;
+        const uint64_t bal = __ballot(tie);
+        __syncthreads();  // the previous round's readers of s are done
+        if (lane == 0) s[wave] = (uint32_t)__popcll(bal);
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+        for (int w = 0; w < kSelThreads / 64; ++w) {
+            before += w < wave ? s[w] : 0u;
+            total += s[w];
+        }
+        const uint32_t mine = before + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+        if (tie && mine + 1 == r) *key = slot_key(__uint_as_float(u ^ 0x80000000u), i);
+        if (r <= total) return;
+        r -= total;
+    }
 }
 
 }  // namespace
@@ -614,21 +785,28 @@ struct RewireArgs {
     const int64_t* key_thr;
 };
 
-template <int WD, int NPT>
-void launch_whole(const RewireArgs& a, int64_t Gc, hipStream_t st) {
-    const void* fn = reinterpret_cast<const void*>(&rewire_whole_kernel<WD, NPT>);
+template <int WD, int NPT, bool GIVEN>
+void launch_whole_s(const RewireArgs& a, int64_t Gc, hipStream_t st) {
+    const void* fn = reinterpret_cast<const void*>(&rewire_whole_kernel<WD, NPT, GIVEN>);
     const int lds = kMiscBytes + (int)(a.G * a.F * El<WD>::es);
-    rewire_whole_kernel<WD, NPT><<<dim3((unsigned)persistent_grid(fn, lds, Gc)), dim3(kThreads),
-                                   lds, st>>>(
+    rewire_whole_kernel<WD, NPT, GIVEN><<<dim3((unsigned)persistent_grid(fn, lds, Gc)),
+                                          dim3(kThreads), lds, st>>>(
         a.W, a.idx, a.scores_out, a.n_pruned, a.O, (int)a.F, (int)a.G, (int)a.D, a.prune_mode,
         a.thr, (int)a.k, a.regrow_mode, a.init_mode, a.bound, (uint32_t)a.seed,
-        (uint32_t)(a.seed >> 32), a.score_mode, Gc);
+        (uint32_t)(a.seed >> 32), a.score_mode, a.scores_in, a.key_thr, Gc);
+}
+template <int WD, int NPT>
+void launch_whole(const RewireArgs& a, int64_t Gc, hipStream_t st) {
+    if (a.scores_in != nullptr)
+        launch_whole_s<WD, NPT, true>(a, Gc, st);
+    else
+        launch_whole_s<WD, NPT, false>(a, Gc, st);
 }
 
 template <int WD>
 void launch_rewire(const RewireArgs& a, int64_t Gc, hipStream_t st) {
     const int es = El<WD>::es;
-    if (a.scores_in == nullptr && a.grad == nullptr && (a.F * es) % 16 == 0 &&
+    if ((a.scores_in != nullptr || a.grad == nullptr) && (a.F * es) % 16 == 0 &&
         a.G * a.F * es <= kStageMax && aligned16(a.W)) {
         switch ((int)((a.G * a.F * es + 16 * kThreads - 1) / (16 * kThreads))) {
             case 1: launch_whole<WD, 1>(a, Gc, st); break;
@@ -743,6 +921,34 @@ extern "C" int haste_rewire_scores(const void* W, int32_t w_dtype, const void* g
         HASTE_RS_LAUNCH(HASTE_DTYPE_F32);
 #undef HASTE_RS_LAUNCH
     HASTE_CHECK_LAUNCH("haste_rewire_scores");
+    return HASTE_OK;
+}
+
+extern "C" int64_t haste_rewire_select_workspace_size(void) {
+    return haste::kSelWords * (int64_t)sizeof(uint32_t);
+}
+
+extern "C" int haste_rewire_select(const float* scores, int64_t n, int64_t k, int64_t* key,
+                                   void* workspace, int64_t ws_bytes, void* stream) {
+    HASTE_CHECK_ARG(scores && key && workspace, "haste_rewire_select: null pointer");
+    HASTE_CHECK_ARG(n >= 1 && n < ((int64_t)1 << 32) && k >= 1 && k <= n,
+                    "haste_rewire_select: invalid n=%lld, k=%lld", (long long)n, (long long)k);
+    HASTE_CHECK_ARG(ws_bytes >= haste_rewire_select_workspace_size(),
+                    "haste_rewire_select: workspace too small (%lld < %lld bytes)",
+                    (long long)ws_bytes, (long long)haste_rewire_select_workspace_size());
+    using namespace haste;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint32_t* ws = static_cast<uint32_t*>(workspace);
+    // 8 scores per thread: fewer workgroups than that add little to a pass's time,
+    // more add their histograms' atomics
+    const unsigned grid = (unsigned)std::min<int64_t>(kSelChunks, ceil_div(n, 8 * kThreads));
+    const int64_t chunk = ceil_div(n, kSelChunks);
+    select_pass_kernel<0><<<dim3(grid), dim3(kThreads), 0, st>>>(scores, n, (uint32_t)k, ws);
+    select_pass_kernel<1><<<dim3(grid), dim3(kThreads), 0, st>>>(scores, n, (uint32_t)k, ws);
+    select_pass_kernel<2><<<dim3(grid), dim3(kThreads), 0, st>>>(scores, n, (uint32_t)k, ws);
+    select_ties_kernel<<<dim3(kSelChunks), dim3(kThreads), 0, st>>>(scores, n, chunk, (uint32_t)k, ws);
+    select_key_kernel<<<dim3(1), dim3(kSelThreads), 0, st>>>(scores, n, chunk, ws, key);
+    HASTE_CHECK_LAUNCH("haste_rewire_select");
     return HASTE_OK;
 }
 

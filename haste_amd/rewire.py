@@ -155,7 +155,7 @@ class GroupFixedFanInReal(GroupFixedFanIn):
         to the lower slot), ``"threshold"`` every score below the threshold;
       * regrowth and initialisation as GroupFixedFanIn (Philox streams keyed by one
         seed per call; ``regrow_mode="unused"`` is also available).
-    Runs as two kernels and one device-side k-th-value selection, no host sync."""
+    Runs on the device (scores, the k-th smallest key, prune and regrow), no host sync."""
 
     def __init__(self, in_features: int, out_features: int, fan_in: int, bias: bool = True,
                  device=None, dtype=None, *, group_size=32, prune_mode="threshold",
@@ -203,11 +203,12 @@ class GroupFixedFanInReal(GroupFixedFanIn):
             scores = torch.empty(Gc, F, dtype=torch.float32, device=W.device)
             _lib.call("haste_rewire_scores", W.data_ptr(), wcode, gptr, gcode, smode,
                       scores.data_ptr(), O, F, G, st)
-            # unique keys (scores are >= 0, so their bits order them): the k-th
-            # smallest is the last pruned slot; ties go to the lower slot
-            keys = (scores.view(-1).view(torch.int32).to(torch.int64) << 32) | torch.arange(
-                Gc * F, dtype=torch.int64, device=W.device)
-            key_thr = torch.kthvalue(keys, k).values.contiguous()
+            # the key (score bits, slot) of the last pruned slot; ties go to the lower slot
+            n = _lib.lib().haste_rewire_select_workspace_size()
+            buf = torch.zeros(1 + (n + 7) // 8, dtype=torch.int64, device=W.device)
+            key_thr, ws = buf[:1], buf[1:]
+            _lib.call("haste_rewire_select", scores.data_ptr(), Gc * F, k, key_thr.data_ptr(),
+                      ws.data_ptr(), n, st)
         if seed is None:
             seed = int(torch.randint(0, 2**62, (1,), dtype=torch.int64).item())
         if self._pruned_total is None or self._pruned_total.device != W.device:

@@ -464,9 +464,15 @@ int haste_rewire(void* W, int32_t w_dtype, int32_t* idx, float* scores_out, int3
  * mode, HASTE_PRUNE_GLOBAL_FRACTION: prune the slots whose key
  * (bits(score) << 32 | g*F + j) is <= *key_thr, the k-th smallest key of the
  * layer (so exactly k slots, the smallest scores, ties to the lower slot),
- * selected by the caller on the device from scores_in (the scores of
- * haste_rewire_scores with the same modes).  Regrow and init as haste_rewire.
+ * selected on the device from scores_in (the scores of haste_rewire_scores with
+ * the same modes), as haste_rewire_select does.  Regrow and init as haste_rewire.
+ * haste_rewire_select writes that key: the k-th smallest (1 <= k <= n) of the n
+ * slots of scores, with no host synchronisation.  Its workspace
+ * (haste_rewire_select_workspace_size bytes, 4-byte aligned) must be zero.
  */
+int64_t haste_rewire_select_workspace_size(void);
+int haste_rewire_select(const float* scores, int64_t n, int64_t k, int64_t* key, void* workspace,
+                        int64_t ws_bytes, void* stream);
 int haste_rewire_scores(const void* W, int32_t w_dtype, const void* grad, int32_t grad_dtype,
                         int32_t score_mode, float* scores, int64_t O, int64_t F, int64_t G,
                         void* stream);
