@@ -58,6 +58,15 @@ struct StagedCfg {
     // groups of load look-ahead; G = 128 fragments are four times larger
     static constexpr int DEPTH = G >= 128 ? 2 : 5;
     static constexpr int NS = DEPTH + 1;     // register slots of the pipeline
+    // read a group's dY operands an iteration early, so that its MFMAs do not
+    // wait on LDS (the registers of the largest operand set, G = 128 at 64 rows,
+    // do not allow it): 94.4 -> 90 us at 111,395 labels, G = 64, F = 192, B = 288,
+    // 73.5 -> 72.8 at 131,073 labels, F = 128, B = 512.  A tile is then staged one
+    // group earlier too: between its store and its reads, and between its
+    // buffer's last reads and the next store, lie three iterations, one of
+    // which ends with the window's barrier.
+    static constexpr bool EARLY = MT * KS <= 8;
+    static constexpr int AHEAD = kPlanWindow + (EARLY ? 1 : 0);
     static_assert(G >= 32, "staged build: G >= 32");
     static_assert(TPW * W == kStagedTiles, "tiles per wave");
     static_assert(PB == 4 || PB == 8 || PB == 16 || PB == 32, "dY piece");
@@ -354,32 +363,35 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
             u32x2 m0[DEPTH + 1];
 #pragma unroll
             for (int k = 0; k <= DEPTH; ++k) m0[k] = load_meta(k);
-            Piece y0[kPlanWindow];
+            Piece y0[C::AHEAD];
 #pragma unroll
-            for (int k = 0; k < kPlanWindow; ++k) y0[k] = load_y(k);
+            for (int k = 0; k < C::AHEAD; ++k) y0[k] = load_y(k);
             for (int k = tid * 4; k < dn * AS; k += NTH * 4)
                 *reinterpret_cast<f32x4*>(&acc[k]) = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 0; k <= DEPTH; ++k) mu[k] = uniform_meta(m0[k]);
 #pragma unroll
-            for (int k = 0; k < kPlanWindow; ++k) stage(k, y0[k], k);
+            for (int k = 0; k < C::AHEAD; ++k) stage(k, y0[k], k);
 #pragma unroll
             for (int k = 0; k < DEPTH; ++k) {
                 __builtin_amdgcn_sched_barrier(0);
                 load_frag(k, mu[k], fq[k % NS]);
-                yq[k % NS] = load_y(k + kPlanWindow);
+                yq[k % NS] = load_y(k + C::AHEAD);
                 mraw[k % NS] = load_meta(k + DEPTH + 1);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_waitcnt(wait_lgkmcnt(0));
         __builtin_amdgcn_s_barrier();
+        // dY operands of groups i (multiplied in iteration i) and i + 1 (read in it)
+        u32x4 aq[C::EARLY ? 2 : 1][MT][KS];
+        if constexpr (C::EARLY) read_a(0, aq[0]);
         auto body = [&](int i, auto kc) __attribute__((always_inline)) {
             constexpr int K = decltype(kc)::value;  // i % kGroupUnroll
             constexpr int Q = K % NS;               // slot of step i
             constexpr int QN = (Q + DEPTH) % NS;    // slot of step i + DEPTH
             load_frag(i + DEPTH, mu[DEPTH], fq[QN]);
-            yq[QN] = load_y(i + DEPTH + kPlanWindow);
+            yq[QN] = load_y(i + DEPTH + C::AHEAD);
             mraw[QN] = load_meta(i + 2 * DEPTH + 1);
             const u32x2 m = mu[0];
             const int tb = (int)(m[0] & 0xFFFF), te = (int)m[1];
@@ -394,12 +406,12 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
                     old[k][mt] = *reinterpret_cast<const f32x4*>(accb + pass1(fod[k]) + mt * 64 + colb);
-            stage(i + kPlanWindow, yq[Q], (K + kPlanWindow) % kStageBufs);
+            stage(i + C::AHEAD, yq[Q], (K + C::AHEAD) % kStageBufs);
             f32x4 pc[TPW][MT];
-            u32x4 a[MT][KS];
-            read_a(K % kStageBufs, a);
+            if constexpr (C::EARLY) read_a((K + 1) % kStageBufs, aq[(K + 1) % 2]);
+            else read_a(K % kStageBufs, aq[0]);
 #pragma unroll
-            for (int k = 0; k < TPW; ++k) mma(a, fq[Q].b0[k], pc[k]);
+            for (int k = 0; k < TPW; ++k) mma(aq[C::EARLY ? K % 2 : 0], fq[Q].b0[k], pc[k]);
 #pragma unroll
             for (int k = 0; k < TPW; ++k) {
                 if (wave + k * WAVES < n0d) {  // uniform: the wave had tile k
