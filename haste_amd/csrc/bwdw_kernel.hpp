@@ -32,6 +32,15 @@
 //    and/or, in the fused mode, applied to W in place by the SGD step of
 //    haste_sgd_sr_step (same FMA chain, same Philox offsets l*F + j for W and l
 //    for the bias), so the fp32 gradient need not make a round trip to HBM.
+//  - FWD (fused mode only): the launch also computes the logits from the weights
+//    before their update, for a step whose dY does not depend on them.  The
+//    forward kernel reads the same weights, indices and gathered rows per
+//    group, and its time goes to writing the logits, this kernel's to reading
+//    dY and to the Philox draws; in one launch they overlap, and one start-up
+//    chain per group is gone.  Two kernels -> one, in the training step: 54 + 76
+//    -> 118 us at O = 131,073, G = 64, F = 128, B = 512; 222 + 235 -> 396 at
+//    O = 670,091, F = 64; 242 + 443 -> 623 at G = 32, F = 256, D = 4096,
+//    O = 500,000, B = 256; 1881 + 2127 -> 3499 at O = 3M, G = F = 128, B = 1024.
 #include <algorithm>
 #include <type_traits>
 
@@ -60,6 +69,8 @@ struct SgdArgs {
     int ndr, Tcap;
     ReduceJob rj;  // ntiles > 0: workgroups Gc .. Gc + ntiles - 1 run this job's tiles
     const uint64_t* seed_dev;  // not NULL: the Philox seed is read here (k0, k1 unused)
+    uint16_t* logits;  // FWD launches: the logits [B, ldl]
+    int64_t ldl;
 };
 
 namespace {
@@ -67,7 +78,8 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kStgBytes = 34 * 1024;  // LDS for one pass of the staged gradient tile
 
-template <int G, int FP>
+// FWD: the launch also computes the logits (see ffi_bwd_w_kernel).
+template <int G, int FP, bool FWD = false>
 struct BwdWCfg {
     // batch rows per LDS stage: 32 at G = 32, F = 256, whose smaller stages then
     // fit four workgroups per CU (LDS and registers), else 64
@@ -91,12 +103,24 @@ struct BwdWCfg {
     // (G = 64, F = 128, whose four waves per SIMD leave 128 registers: the
     // staging there spilled one), and 2132 -> 2164 at config 4 (G = 128).  Those
     // two keep the fragment loads.
-    static constexpr bool XS = G <= 64 && !(G == 64 && FP == 128);
+    // FWD: always (the forward reads the same rows).
+    static constexpr bool XS = FWD || (G <= 64 && !(G == 64 && FP == 128));
     static constexpr int RBX = KC * 2 + 16;                  // LDS bytes per staged X^T row
     static constexpr int XS_BYTES = XS ? FP * RBX : 0;        // one chunk of the gathered rows
     static constexpr int PPTX = FP * (KC / 8) / kThreads;    // X^T pieces per thread
     static constexpr int STG_BYTES = PR * SP * 4;
-    static constexpr int LDS_BYTES = YS_BYTES + XS_BYTES > STG_BYTES ? YS_BYTES + XS_BYTES : STG_BYTES;
+    // FWD: label waves (a wave keeps at most eight weight fragments, 32
+    // registers, where four waves allow it; four at G = 64, F = 128, which
+    // spilled 18 registers at three waves per SIMD otherwise), label tiles and
+    // column blocks per wave, and the staged logits of a chunk
+    static constexpr int KSF = FP / 32;
+    static constexpr int WMF = NTILES * KSF <= 8 ? 1 : NTILES * KSF <= 16 && NTILES >= 2 && !(G == 64 && FP == 128) ? 2
+                               : NTILES >= 4 ? 4 : NTILES;
+    static constexpr int MTF = NTILES / WMF, NTF = KC / 16 * WMF / 4;
+    static constexpr int RBF = 2 * G + 16;
+    static constexpr int FS_BYTES = FWD ? KC * RBF : 0;
+    static constexpr int LOOP_BYTES = YS_BYTES + XS_BYTES + FS_BYTES;
+    static constexpr int LDS_BYTES = LOOP_BYTES > STG_BYTES ? LOOP_BYTES : STG_BYTES;
     static constexpr int CPR = FP / 8;                        // 8-slot chunks per staged row
     static constexpr int WPT = (PR * CPR + kThreads - 1) / kThreads;  // chunks per thread, pass 0
     static_assert(PR >= 16 && G % PR == 0, "epilogue pass shape");
@@ -124,8 +148,9 @@ __device__ __forceinline__ u32x4 keep_first(u32x4 v, int nv) {
 // G = 64, FP = 128 four fit (the fused update then loads W in its epilogue):
 // the 2049 groups of a 131K-label layer run in two rounds of 1024, not three
 // of 768.
-template <int G, int FP>
+template <int G, int FP, bool FWD = false>
 constexpr int bwdw_waves_per_simd() {
+    if (FWD) return G <= 64 && G * FP <= 64 * 128 ? 3 : 2;
     return (G == 64 && FP == 128) || (G == 32 && FP == 256) ? 4 : G * FP >= 128 * 256 ? 1 : 2;
 }
 
@@ -134,18 +159,19 @@ constexpr int bwdw_waves_per_simd() {
 // does not evict the weights that the next step's forward reads.
 constexpr int kLoadNT = 2;  // buffer-load cache policy: nt on gfx950
 
-template <typename T, int G, int FP, bool SGD, bool YNT, bool YS>
-__global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_bwd_w_kernel(
+template <typename T, int G, int FP, bool SGD, bool YNT, bool YS, bool FWD>
+__global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP, FWD>())) void ffi_bwd_w_kernel(
     const int32_t* __restrict__ idx, const uint16_t* __restrict__ xT, int64_t ldx,
     const uint16_t* __restrict__ dY, int64_t lddy, void* __restrict__ dW, int dW_dtype,
     void* __restrict__ dbias, int dbias_dtype, int B, int D, int F, int64_t O, SgdArgs sg) {
     constexpr bool yshort = YS;
-    using C = BwdWCfg<G, FP>;
+    using C = BwdWCfg<G, FP, FWD>;
     constexpr int MT = C::MT, NT = C::NT, RB = C::RB, PPT = C::PPT, SP = C::SP, PR = C::PR;
     constexpr bool XS = C::XS;
     constexpr int RBX = C::RBX, PPTX = XS ? C::PPTX : 1, KC = C::KC, KSC = KC / 32;
     __shared__ __attribute__((aligned(16))) char lds[C::LDS_BYTES];
     __shared__ int s_perm[SGD ? FP : 1];
+    __shared__ __attribute__((aligned(16))) float s_fb[FWD ? G : 1];  // FWD: the bias
     __shared__ float s_bg[SGD ? G : 1];  // fused step: the bias gradient of the group
     char (*Ys)[KC * RB] = reinterpret_cast<char (*)[KC * RB]>(lds);
     char* Xs = lds + C::YS_BYTES;
@@ -287,6 +313,69 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
         }
     };
 
+    // FWD: the logits' operands.  A: W fragments of the wave's label tiles
+    // (labels past O and slots past F read as zero); B: the staged rows.
+    constexpr int KSF = C::KSF, MTF = C::MTF, NTF = C::NTF, RBF = C::RBF;
+    const int wmf = wave % C::WMF, wnf = wave / C::WMF;
+    char* Fs = lds + C::YS_BYTES + C::XS_BYTES;
+    u32x4 wf[FWD ? MTF : 1][FWD ? KSF : 1];
+    if constexpr (FWD) {
+        const rsrc_t fwr = make_rsrc(sg.W + l0 * F, (int64_t)nl * F * 2);
+#pragma unroll
+        for (int mt = 0; mt < MTF; ++mt) {
+#pragma unroll
+            for (int ks = 0; ks < KSF; ++ks) {
+                const int k = ks * 32 + kq * 8;
+                wf[mt][ks] = buf_load16(
+                    fwr, k < F ? (uint32_t)(((wmf * MTF + mt) * 16 + col) * F + k) * 2 : kOOB);
+            }
+        }
+    }
+    // logits of chunk c from the staged rows, rounded, into Fs [64 rows][G]
+    auto fwd_chunk = [&]() {
+#pragma unroll
+        for (int nt = 0; nt < NTF; ++nt) {
+            const int n0 = (wnf * NTF + nt) * 16;
+            f32x4 a[MTF];
+#pragma unroll
+            for (int mt = 0; mt < MTF; ++mt) a[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KSF; ++ks) {
+                const char* p = Xs + (ks * 32 + kq * 8 + col / 4) * RBX + (col % 4) * 8 + n0 * 2;
+                const u32x2 lo = lds_read_tr16(p);
+                const u32x2 hi = lds_read_tr16(p + 4 * RBX);
+                const u32x4 bf = u32x4{lo[0], lo[1], hi[0], hi[1]};
+#pragma unroll
+                for (int mt = 0; mt < MTF; ++mt) a[mt] = mfma16x16x32<T>(wf[mt][ks], bf, a[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MTF; ++mt) {
+                const int lb = (wmf * MTF + mt) * 16 + kq * 4;
+                const f32x4 v = a[mt] + *reinterpret_cast<const f32x4*>(&s_fb[lb]);
+                *reinterpret_cast<u32x2*>(Fs + (n0 + col) * RBF + lb * 2) =
+                    u32x2{pack2_rne<T>(v[0], v[1]), pack2_rne<T>(v[2], v[3])};
+            }
+        }
+    };
+    // the staged logits of chunk c as whole rows of the group
+    auto fwd_flush = [&](int c) {
+        constexpr int LPR = G / 8, RPI = 64 / LPR;  // lanes per row, rows per instruction
+        constexpr int RPW = KC / 4;                 // rows per wave
+        const int b0 = c * KC, rows = std::min(KC, B - b0);
+        const rsrc_t lr = make_rsrc(sg.logits + (int64_t)b0 * sg.ldl + l0,
+                                    ((int64_t)(rows - 1) * sg.ldl + (nl + 7) / 8 * 8) * 2);
+        // a store with every lane out of range may retire ahead of older loads
+        if (rows < KC || nl < G) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+#pragma unroll
+        for (int r0 = 0; r0 < RPW; r0 += RPI) {
+            const int rr = wave * RPW + r0 + lane / LPR, cl = (lane % LPR) * 8;
+            const bool own = (RPI <= RPW || lane / LPR < RPW) && rr < rows && cl < nl;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(Fs + (own ? rr : 0) * RBF + cl * 2);
+            __builtin_amdgcn_raw_buffer_store_b128(
+                v, lr, own ? (uint32_t)(rr * (uint32_t)sg.ldl + cl) * 2 : kOOB, 0, kLoadNT);
+        }
+    };
+
     // The bias MFMA of label tile nt runs on the wave with wm == nt % WM, into
     // its accumulator accb[nt / WM]: the waves share the work and hold
     // ceil(NT / WM) accumulators each, not NT.
@@ -312,7 +401,7 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
     // .. +7).  For at most two passes and F <= 128: beyond that the extra
     // registers would cost a wave per SIMD (so would they at four waves).
     constexpr int NPASS = G / PR;
-    constexpr bool kWPre = SGD && NPASS <= 2 && FP <= 128 && bwdw_waves_per_simd<G, FP>() < 4;
+    constexpr bool kWPre = SGD && !FWD && NPASS <= 2 && FP <= 128 && bwdw_waves_per_simd<G, FP>() < 4;
     u32x4 wpre[kWPre ? NPASS * WPT : 1];
     uint32_t bpre = 0;  // fused step: bias bits of label tid (tid < nl)
     if constexpr (SGD) {
@@ -339,6 +428,9 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
     u32x4 yr[2][PPT];
     u32x4 ar[XS ? 1 : 2][KSC][MT];
     u32x4 xv[PPTX];
+    if constexpr (FWD) {
+        if (tid < G) s_fb[tid] = bits_to_f32<T>(bpre);
+    }
     fetch(0, yr[0]);
     fetch(1, yr[1]);
     if constexpr (XS) fetch_x(0, xv);
@@ -357,7 +449,8 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
     auto body = [&](int c, auto parity) {
         constexpr int P = decltype(parity)::value;
         if constexpr (!XS) fetch_a(c + 1, ar[1 - P]);
-        if (active && c < nchunks) {
+        if constexpr (FWD) fwd_chunk();
+        if (active && (FWD || c < nchunks)) {
             const char* ys = Ys[P];
 #pragma unroll
             for (int ks = 0; ks < KSC; ++ks) {
@@ -392,10 +485,12 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
         }
         stash(c + 1, 1 - P, yr[1 - P]);  // chunk c + 1 (zeros past the end)
         fetch(c + 3, yr[1 - P]);
+        if constexpr (FWD) fwd_flush(c);
         __syncthreads();
     };
     for (int c = 0; c < nchunks; c += 2) {
         body(c, std::integral_constant<int, 0>{});
+        if (FWD && c + 1 >= nchunks) break;
         body(c + 1, std::integral_constant<int, 1>{});
     }
 
@@ -566,18 +661,18 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP>())) void ffi_
     }
 }
 
-template <typename T, int G, int FP, bool SGD, bool YNT, bool YS>
+template <typename T, int G, int FP, bool SGD, bool YNT, bool YS, bool FWD = false>
 int launch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16_t* dY, int64_t lddy,
            void* dW, int dW_dtype, void* dbias, int dbias_dtype, int64_t B, int64_t D, int64_t F,
            int64_t O, const SgdArgs& sg, hipStream_t st) {
     const int64_t Gc = ceil_div(O, G);
     if (Gc + sg.rj.ntiles > 0x7FFFFFFF || D * ldx * 2 > kMaxRsrcBytes ||
-        ((int64_t)BwdWCfg<G, FP>::KC * lddy + 8) * 2 > kMaxRsrcBytes || (int64_t)G * F * 4 > kMaxRsrcBytes) {
+        ((int64_t)BwdWCfg<G, FP, FWD>::KC * lddy + 8) * 2 > kMaxRsrcBytes || (int64_t)G * F * 4 > kMaxRsrcBytes) {
         set_error("haste_ffi_bwd_weights: problem too large (Gc %lld, lddy %lld, D*ldx %lld)",
                   (long long)Gc, (long long)lddy, (long long)(D * ldx));
         return HASTE_ERR_UNSUPPORTED;
     }
-    ffi_bwd_w_kernel<T, G, FP, SGD, YNT, YS><<<dim3((unsigned)(Gc + sg.rj.ntiles)), dim3(kThreads), 0, st>>>(
+    ffi_bwd_w_kernel<T, G, FP, SGD, YNT, YS, FWD><<<dim3((unsigned)(Gc + sg.rj.ntiles)), dim3(kThreads), 0, st>>>(
         idx, xT, ldx, dY, lddy, dW, dW_dtype, dbias, dbias_dtype, (int)B, (int)D, (int)F, O, sg);
     HASTE_CHECK_LAUNCH("haste_ffi_bwd_weights");
     return HASTE_OK;
@@ -611,6 +706,13 @@ int dispatch_g(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16
 }
 
 }  // namespace
+
+// The SGD launch that also computes the logits (FWD kernels; defined in
+// ffi_forward_bwdw.hip), for the dY, logits stride and tile sizes it has builds for.
+bool fwd_sgd_fits(const void* dY, int64_t lddy, int64_t ldl, int64_t F, int64_t G);
+int fwd_sgd_dispatch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16_t* dY,
+                     int64_t lddy, int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
+                     const SgdArgs& sg, hipStream_t st);
 
 // dY rows at a stride that is not a multiple of 8 (YS kernels; defined in
 // ffi_bwd_weights_ys.hip).  Same arguments as the dispatch of ffi_bwd_weights.hip.

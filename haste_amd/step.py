@@ -114,8 +114,7 @@ class FFITrainStep:
     def logits(self) -> torch.Tensor:
         return self.logits_buf[:, : self.O]
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        """x [B, D] bf16 -> logits [B, O] (view of a [B, ldo] buffer)."""
+    def _load_features(self, x: torch.Tensor) -> None:
         if tuple(x.shape) != (self.B, self.D) or x.dtype != torch.bfloat16:
             raise ValueError(f"FFITrainStep.forward: x must be bf16 [{self.B}, {self.D}] "
                              f"(got {x.dtype} {list(x.shape)})")
@@ -124,6 +123,10 @@ class FFITrainStep:
             x = x.contiguous()
         _lib.call("haste_transpose_features", x.data_ptr(), x.stride(0), self.xT_buf.data_ptr(),
                   self.ldx, self.B, self.D, _C.stream_of(self.W))
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        """x [B, D] bf16 -> logits [B, O] (view of a [B, ldo] buffer)."""
+        self._load_features(x)
         _lib.call("haste_ffi_forward", self.idx.data_ptr(), self.xT_buf.data_ptr(), self.ldx,
                   self.W.data_ptr(), None if self.bias is None else self.bias.data_ptr(),
                   self.logits_buf.data_ptr(), self.ldo, self.B, self.D, self.F, self.O, self.G,
@@ -282,16 +285,39 @@ class FFITrainStep:
                       self.seed, self.ws.data_ptr() if plan_ok else None,
                       self.ws.numel() if plan_ok else 0, self.B, self.D, self.F, self.O, self.G,
                       self.code, _C.stream_of(self.W))
+        self._weights_updated(plan_ok)
+
+    def _weights_updated(self, wt: bool) -> None:
         # the kernel wrote W in place: move torch's version counter, as an in-place
         # torch op would, and record that the workspace holds W^T of this version
         torch.autograd.graph.increment_version(self.W)
-        self._wt_version = self.W._version if plan_ok else None
+        self._wt_version = self.W._version if wt else None
         if self._seed_dev is None:
             self.seed += 1
 
     def step(self, x: torch.Tensor, dY: torch.Tensor, lddy: int) -> None:
-        """forward -> backward to features (partials) -> fused weight/bias gradient +
-        SR-SGD, whose launch also finishes dX."""
-        self.forward(x)
+        """Forward, backward to features (partials) and the fused weight/bias gradient +
+        SR-SGD, whose launch also finishes dX.  dY is given, so the logits need
+        not come first: they are computed in the update's launch too, from the
+        weights and features it reads anyway (haste_ffi_forward_bwd_weights_sgd_dx;
+        bit-identical to forward, backward_features, backward_weights_sgd in turn).
+        A dY that shares memory with the logits is read after they are written."""
+        lo, hi = self.logits_buf.data_ptr(), dY.data_ptr()
+        if (self.grad_dtype != torch.float32 or (hi < lo + self.logits_buf.numel() * 2
+                                                 and lo < hi + dY.numel() * dY.element_size())):
+            self.forward(x)
+            self.backward_features(dY, lddy, defer_dx=True)
+            self.backward_weights_sgd(dY, lddy)
+            return
+        self._load_features(x)
         self.backward_features(dY, lddy, defer_dx=True)
-        self.backward_weights_sgd(dY, lddy)
+        seed_dev = None if self._seed_dev is None else self._seed_dev.data_ptr()
+        _lib.call("haste_ffi_forward_bwd_weights_sgd_dx", self.idx.data_ptr(),
+                  self.xT_buf.data_ptr(), self.ldx, dY.data_ptr(), lddy, self.W.data_ptr(),
+                  None if self.bias is None else self.bias.data_ptr(), None, None,
+                  self.logits_buf.data_ptr(), self.ldo, self.lr, self.wd, 0.0, 0, 1, self.seed,
+                  seed_dev, self.dX.data_ptr(), SR_SEED_GRAD_X, self.ws.data_ptr(),
+                  self.ws.numel(), self.B, self.D, self.F, self.O, self.G, self.code,
+                  _C.stream_of(self.W))
+        self._dx_pending = False
+        self._weights_updated(True)

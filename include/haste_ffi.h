@@ -325,6 +325,24 @@ int haste_sgd_sr_step_wt(uint16_t* W, const void* g, int32_t g_dtype, float* m, 
                          int64_t O, int64_t G, int32_t dtype, void* stream);
 
 /*
+ * haste_ffi_forward with the weights and bias as they are on entry, and
+ * haste_ffi_bwd_weights_sgd_dx (seed_dev not NULL: ..._dev_seed, seed unused), in
+ * one launch where the sizes have a build for it (rows of dY on 16-byte
+ * boundaries, G * F up to 128 * 128 or G < 128), else one after the other: for a
+ * step whose dY does not depend on these logits, which reads each group's
+ * weights and gathered features once instead of twice.  logits: [B, ldl] bf16,
+ * ldl >= O and a multiple of 8, 16-byte aligned, must not overlap dY; the columns
+ * from O up to the next multiple of 8 may be overwritten.  Bit-identical to the
+ * two calls.  The bwd-features call comes first (before this call's update of W).
+ */
+int haste_ffi_forward_bwd_weights_sgd_dx(
+    const int32_t* idx, const void* xT, int64_t ldx, const void* dY, int64_t lddy, uint16_t* W,
+    uint16_t* bias, float* m_W, float* m_bias, uint16_t* logits, int64_t ldl, float lr, float wd,
+    float mu, int32_t use_mom, int32_t do_sr, uint64_t seed, uint64_t* seed_dev, uint16_t* dX,
+    uint64_t dx_seed, void* bwdf_workspace, int64_t bwdf_workspace_bytes, int64_t B, int64_t D,
+    int64_t F, int64_t O, int64_t G, int32_t dtype, void* stream);
+
+/*
  * haste_sgd_sr_step_wt that also steps the layer's bias [O] (bf16) with its
  * gradient gb [O] (bf16, f16 or f32) and fp32 momentum m_bias (read and written
  * when use_mom), in the same launch: the same update as haste_sgd_sr_step on
