@@ -128,6 +128,7 @@ struct BwdFPlan {
     int64_t Gc, BT, nbt, Bp, ndr, Dc, S, gps, Tcap;
     int64_t RT, DCMAX;  // ring tiles of the main kernel; its partial's trash rows start at DCMAX
     int64_t staged;     // the plan is for the staged main kernel (RT unused)
+    int64_t tiles;      // its pipeline tiles: kStagedTiles, or half as many, two waves to a tile
     int64_t tfeat_off, tsrc_off, perm_off, meta_off, twt_off, prep_bytes, ws_bytes;
 };
 
@@ -241,6 +242,10 @@ inline BwdFPlan make_plan_for(int64_t B, int64_t D, int64_t F, int64_t O, int64_
     p.nbt = ceil_div(B, p.BT);
     p.Bp = p.nbt * p.BT;
     p.ndr = ceil_div(D, p.DCMAX);
+    p.tiles = kStagedTiles;
+    if (p.staged && F > (p.ndr == 1 ? 48 : 32 * p.ndr) &&
+        ring_overflow(F, 1.0 / (double)p.ndr, kStagedTiles / 2) < 0.01)
+        p.tiles = kStagedTiles / 2;
     p.Dc = ceil_div(D, p.ndr);
     int64_t S = std::max<int64_t>(1, kTargetCTAs / (p.nbt * p.ndr));
     S = std::min<int64_t>(S, std::max<int64_t>(1, ceil_div(p.Gc, 8)));
@@ -268,14 +273,19 @@ inline BwdFPlan make_plan_for(int64_t B, int64_t D, int64_t F, int64_t O, int64_
 // where a group's range holds seven or more tiles of 16 positions, so that
 // nearly all of its eight waves have a tile (measured, config 1: 86 -> 82 us;
 // config 4: 3452 -> 2402 us; with four tiles, configs 2 and 3, it was slower
-// than the ring and direct builds: 295 -> 336 and 606 -> 805 us), and where
-// the slice's W^T tiles span at most kMaxRsrcBytes (its 32-bit tile offsets).
+// than the ring and direct builds: 295 -> 336 and 606 -> 805 us).  With two
+// waves to a tile it is the faster one for ranges of at most four tiles, too,
+// measured: 345 -> 300 us at O = 670,091, G = F = 64, B = 512, D = 768; 185 -> 157
+// (two ranges: G = 64, F = 96, D = 1500, O = 300,000, B = 256); 212 -> 202 (G = 32,
+// F = 80, D = 1700); 104 -> 51 (fp32 layer, G = 32, F = 64, B = 256, O = 131,073);
+// three tiles in one range (F = 48) were slower: 202 -> 206.  Either way the slice's
+// W^T tiles must span at most kMaxRsrcBytes (its 32-bit tile offsets).
 inline BwdFPlan make_plan(int64_t B, int64_t D, int64_t F, int64_t O, int64_t G) {
     const int build = bwdf_build();
     if (G >= 32 && (build == 0 || build == 3)) {
         const BwdFPlan p = make_plan_for(B, D, F, O, G, true);
         const bool fits = (p.gps + 8) * p.Tcap * 16 * G * 2 <= kMaxRsrcBytes;
-        if (fits && (build == 3 || F >= 7 * 16 * p.ndr)) return p;
+        if (fits && (build == 3 || F >= 7 * 16 * p.ndr || p.tiles < kStagedTiles)) return p;
     }
     return make_plan_for(B, D, F, O, G, false);
 }

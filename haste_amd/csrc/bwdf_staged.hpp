@@ -22,6 +22,8 @@
 //    out windows of kPlanWindow consecutive groups with every feature they
 //    share in the tile of the same index -- one wave -- so the window's
 //    updates need no barrier between them: one barrier per window.
+// A range of at most four tiles (TILES = 4) takes two waves to a tile, each with
+// half of the batch tile's row blocks, so that all eight have work.
 // A duplicated index's second ("lo") row sits in the same tile as its "hi"
 // row (the plan's in-tile mode: no layer-1 tiles, so no wave carries a second
 // tile in the pipeline), its partial-row offset marked by bit 0: the wave adds
@@ -42,13 +44,14 @@
 namespace haste {
 namespace {
 
-template <int G, int BT, int W>
+template <int G, int BT, int W, int TILES>
 struct StagedCfg {
     static constexpr int WAVES = W;
-    static constexpr int TPW = kStagedTiles / W;  // pipeline tiles per wave
+    static constexpr int TPW = TILES >= W ? TILES / W : 1;  // pipeline tiles per wave
+    static constexpr int WPT = TILES >= W ? 1 : W / TILES;  // waves sharing a tile, by row blocks
     static constexpr int NTH = 64 * WAVES;
     static constexpr int KS = G / 32;        // MFMA k-steps over the group's labels
-    static constexpr int MT = BT / 16;       // 16-row blocks of the batch tile
+    static constexpr int MT = BT / 16 / WPT; // 16-row blocks of the batch tile per wave
     static constexpr int RB = 2 * G;         // bytes of a staged dY row
     static constexpr int STG = BT * RB;      // bytes of a staging buffer
     static constexpr int PB = STG / NTH;     // dY bytes each thread loads per group
@@ -68,7 +71,7 @@ struct StagedCfg {
     static constexpr bool EARLY = MT * KS <= 8;
     static constexpr int AHEAD = kPlanWindow + (EARLY ? 1 : 0);
     static_assert(G >= 32, "staged build: G >= 32");
-    static_assert(TPW * W == kStagedTiles, "tiles per wave");
+    static_assert(TPW * W == TILES * WPT && MT * WPT * 16 == BT, "tiles per wave");
     static_assert(PB == 4 || PB == 8 || PB == 16 || PB == 32, "dY piece");
     static_assert(kGroupUnroll % NS == 0 && kGroupUnroll % 2 == 0 && kGroupUnroll % kStageBufs == 0, "unroll");
     static_assert(DCMAX > 0, "LDS budget");
@@ -137,12 +140,12 @@ __device__ __forceinline__ void piece_shift_down(uint32_t (&w)[PW], int sh) {
     for (int k = 0; k < PW; ++k) w[k] = o[k];
 }
 
-template <typename T, int G, int BT, int W, bool YA>
+template <typename T, int G, int BT, int W, int TILES, bool YA>
 __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
     const int* __restrict__ tfeat, const int* __restrict__ meta, const uint16_t* __restrict__ twt,
     const uint16_t* __restrict__ dY, int64_t lddy, float* __restrict__ ws, int B, int Bp, int D,
     int64_t O, int64_t Gc, int nbt, int ndr, int Dc, int gps, int S, int Tcap) {
-    using C = StagedCfg<G, BT, W>;
+    using C = StagedCfg<G, BT, W, TILES>;
     constexpr int KS = C::KS, MT = C::MT, STG = C::STG, PB = C::PB, PW = C::PW, AS = C::AS;
     constexpr int NTH = C::NTH, DEPTH = C::DEPTH, NS = C::NS, WAVES = C::WAVES;
     constexpr int TPW = C::TPW;
@@ -163,6 +166,8 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wt = C::WPT == 1 ? wave : wave % TILES;     // the wave's tile (and every
+    const int mb = C::WPT == 1 ? 0 : wave / TILES * MT;   // WAVES-th after); its first row block
     const int col = lane & 15;  // operand row within a 16-row block / tile position
     const int kq = lane >> 4;   // which 8 of an MFMA's 32 labels
 
@@ -227,13 +232,13 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
                 u32x4{w[4], w[5], w[6], w[7]};
         }
     };
-    // the dY operand fragments of all BT rows from staging buffer buf
+    // the dY operand fragments of the wave's row blocks from staging buffer buf
     auto read_a = [&](int buf, u32x4 (&a)[MT][KS]) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
-                a[mt][ks] = *reinterpret_cast<const u32x4*>(&stg[buf][stg_off<G>(16 * mt + col, 4 * ks + kq)]);
+                a[mt][ks] = *reinterpret_cast<const u32x4*>(&stg[buf][stg_off<G>(16 * (mb + mt) + col, 4 * ks + kq)]);
     };
 
     // ---- per-group metadata: tile range of group g_lo + i in range r, (tb |
@@ -251,7 +256,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
     };
 
     char* const accb = reinterpret_cast<char*>(acc);
-    const int colb = kq * 16;  // bytes: batch rows 4kq .. 4kq+3 of a 16-row block
+    const int colb = mb * 64 + kq * 16;  // bytes: batch rows 4kq .. 4kq+3 of the first row block
 
     // W^T tiles and their partial-row offsets of the slice's groups, addressed by
     // 32-bit offsets from the slice's first tile (the plan keeps a slice's twt
@@ -286,7 +291,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
         auto load_frag = [&](int i, u32x2 m, Frag& fr) __attribute__((always_inline)) {
             const uint32_t tb = m[0] & 0xFFFFu;
             // the wave's tile, counted from the slice's first
-            const uint32_t t0 = (uint32_t)i * (uint32_t)Tcap + tb + (uint32_t)wave;
+            const uint32_t t0 = (uint32_t)i * (uint32_t)Tcap + tb + (uint32_t)wt;
             const uint32_t fl = (uint32_t)lane * 16u;  // the lane's 16 bytes of a k-step's 1 KB
 #pragma unroll
             for (int k = 0; k < TPW; ++k)
@@ -324,9 +329,9 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
                 }
             }
         };
-        // Tiles of group g_lo + i beyond the pipeline's (>= kStagedTiles),
-        // loaded and added at once by the wave that owns the pipeline tile of
-        // the same index modulo WAVES.
+        // Tiles of group g_lo + i beyond the pipeline's (>= TILES), loaded and
+        // added at once by the waves that own the pipeline tile of the same
+        // index modulo the waves' tiles.
         auto extra = [&](int i, u32x2 m, int buf) __attribute__((always_inline)) {
             const int tb = (int)(m[0] & 0xFFFF), te = (int)m[1];
             const int64_t gbase = (g_lo + __builtin_amdgcn_readfirstlane(i)) * Tcap;
@@ -335,7 +340,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
             // tiles are addressed from the group's first tile (all in range)
             const rsrc_t wr = make_rsrc_u32(twt + gbase * 16 * G, (uint32_t)te * 16u * G * 2u);
             const rsrc_t frr = make_rsrc_u32(tfeat + gbase * 16, (uint32_t)te * 16u * 4u);
-            for (int t = wave + kStagedTiles; t < te - tb; t += WAVES) {
+            for (int t = wt + TILES; t < te - tb; t += TILES / TPW) {
                 u32x4 b0[KS];
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks)
@@ -414,7 +419,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
             for (int k = 0; k < TPW; ++k) mma(aq[C::EARLY ? K % 2 : 0], fq[Q].b0[k], pc[k]);
 #pragma unroll
             for (int k = 0; k < TPW; ++k) {
-                if (wave + k * WAVES < n0d) {  // uniform: the wave had tile k
+                if (wt + k * WAVES < n0d) {  // uniform: the wave had tile k
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt)
                         *reinterpret_cast<f32x4*>(accb + pass1(fod[k]) + mt * 64 + colb) = old[k][mt] + pd[k][mt];
@@ -445,7 +450,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
             // the iteration of a window's first group, and of a group the
             // plan could not lay out with its window; a tile staged
             // kPlanWindow groups ahead is published by one of them in time.
-            const bool more = te - tb > kStagedTiles;  // uniform, rare
+            const bool more = te - tb > TILES;  // uniform, rare
             if (K % kPlanWindow == 0 || (m[0] & kMetaUnpaired) || more) {
                 __builtin_amdgcn_s_waitcnt(wait_lgkmcnt(0));
                 __builtin_amdgcn_s_barrier();
@@ -466,7 +471,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
         }
 #pragma unroll
         for (int k = 0; k < TPW; ++k)
-            if (wave + k * WAVES < n0d) add_tile(fod[k], pd[k]);
+            if (wt + k * WAVES < n0d) add_tile(fod[k], pd[k]);
         // every load has been used (the last iterations' look-ahead loads are
         // out of range or unused)
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
@@ -483,7 +488,7 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
     }
 }
 
-template <typename T, int G, int BT, int W, bool YA>
+template <typename T, int G, int BT, int W, int TILES, bool YA>
 int launch_staged(const int* tfeat, const int* meta, const uint16_t* twt, const uint16_t* dY,
                   int64_t lddy, float* ws, const BwdFPlan& p, int64_t B, int64_t D, int64_t O,
                   hipStream_t st) {
@@ -493,7 +498,7 @@ int launch_staged(const int* tfeat, const int* meta, const uint16_t* twt, const 
         set_error("haste_ffi_bwd_features: lddy = %lld too large", (long long)lddy);
         return HASTE_ERR_UNSUPPORTED;
     }
-    bwdf_staged_kernel<T, G, BT, W, YA><<<dim3((unsigned)grid), dim3(64 * W), 0, st>>>(
+    bwdf_staged_kernel<T, G, BT, W, TILES, YA><<<dim3((unsigned)grid), dim3(64 * W), 0, st>>>(
         tfeat, meta, twt, dY, lddy, ws, (int)B, (int)p.Bp, (int)D, O, p.Gc, (int)p.nbt, (int)p.ndr,
         (int)p.Dc, (int)p.gps, (int)p.S, (int)p.Tcap);
     HASTE_CHECK_LAUNCH("haste_ffi_bwd_features");

@@ -234,7 +234,7 @@ struct PlanSlot {
     bool first;
 };
 
-// The analysis of group g's index row by the workgroup's 256 threads: the
+// The analysis of group g's index row by the workgroup's threads: the
 // clamped indices in s_idx (padded to a multiple of 4 slots), first-occurrence /
 // duplicated flags in s_flag, perm, the per-range counts of distinct (s_c[0])
 // and duplicated (s_c[1]) features, and the thread's slot (pn / pd left 0, see
@@ -308,6 +308,7 @@ __device__ __forceinline__ void plan_keys(PlanSlot& ps, int F, int Dc, const int
 // range, meta (tm = te, bit 31 of word 0 = flag), the rows of the thread's
 // feature and the padding rows.  *t_rel receives the tile of the thread's
 // feature relative to its range's first.
+template <int NT>
 __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int F, int ndr, int Tcap,
                                              int row_bytes, int trash_row, uint32_t flag,
                                              int (*s_c)[kMaxRanges], int* s_toff,
@@ -323,7 +324,7 @@ __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int 
         s_toff[ndr] = t;
     }
     __syncthreads();
-    for (int rr = tid; rr < ndr; rr += 256) {
+    for (int rr = tid; rr < ndr; rr += NT) {
         int* m = meta + (g * ndr + rr) * kMetaStride;
         m[0] = (int)((uint32_t)s_toff[rr] | ((uint32_t)s_toff[rr + 1] << 16) | flag);
         m[1] = s_toff[rr + 1];
@@ -348,7 +349,7 @@ __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int 
         }
     }
     const int nslots = s_toff[ndr] * 16;
-    for (int i = tid; i < nslots; i += 256) {
+    for (int i = tid; i < nslots; i += NT) {
         const int t = i / 16, p = i % 16;
         int rr = 0;
         while (t >= s_toff[rr + 1]) ++rr;  // empty ranges are skipped
@@ -422,7 +423,9 @@ __device__ __forceinline__ void pair_range_table(int r, int c0, int nd, int maxp
     *nt = ok ? nt2 : kPairRangeTiles + 1;
 }
 
-__global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __restrict__ idx,
+// NT threads, at least one per slot.
+template <int NT>
+__global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(const int32_t* __restrict__ idx,
                                                                int* __restrict__ tfeat,
                                                                int* __restrict__ tsrc,
                                                                int* __restrict__ perm,
@@ -430,16 +433,16 @@ __global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __
                                                                int ndr, int Dc, int Tcap,
                                                                int row_bytes, int trash_row,
                                                                int64_t Gc) {
-    __shared__ __align__(16) int s_idx[kPlanWindow][256];
-    __shared__ __align__(16) int s_flag[kPlanWindow][256];
-    __shared__ __align__(16) int s_ftile[kPlanWindow][256];   // tile of the slot's feature (first occurrences)
+    __shared__ __align__(16) int s_idx[kPlanWindow][NT];
+    __shared__ __align__(16) int s_flag[kPlanWindow][NT];
+    __shared__ __align__(16) int s_ftile[kPlanWindow][NT];   // tile of the slot's feature (first occurrences)
     __shared__ int s_c[2][kMaxRanges];
     __shared__ int s_toff[kMaxRanges + 1];
     __shared__ int s_pd[kPairRanges][kPairRangeTiles];        // pinned duplicated features per tile
     __shared__ int s_rs[kPairRanges][kPairRangeTiles];        // pinned single features per tile
     __shared__ int s_used[kPairRanges][kPairRangeTiles];      // rows used per tile
     __shared__ int s_maxpin[kPairRanges];
-    __shared__ __align__(16) short s_pin[256];                // the slot's pinned tile, or -1
+    __shared__ __align__(16) short s_pin[NT];                // the slot's pinned tile, or -1
     __shared__ PairTables s_tb;
     __shared__ int s_nt[kPairRanges];                         // tiles per range
     __shared__ int s_fail;
@@ -447,8 +450,8 @@ __global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __
     for (int j = 0; j < kPlanWindow; ++j) {
         const int64_t g = kPlanWindow * (int64_t)blockIdx.x + j;
         if (g >= Gc) return;  // (uniform)
-        for (int i = tid; i < 2 * kMaxRanges; i += 256) (&s_c[0][0])[i] = 0;
-        for (int i = tid; i < kPairRanges * kPairRangeTiles; i += 256) {
+        for (int i = tid; i < 2 * kMaxRanges; i += NT) (&s_c[0][0])[i] = 0;
+        for (int i = tid; i < kPairRanges * kPairRangeTiles; i += NT) {
             (&s_pd[0][0])[i] = 0;
             (&s_rs[0][0])[i] = 0;
             (&s_used[0][0])[i] = 0;
@@ -533,13 +536,13 @@ __global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __
         if (s_fail) {  // (uniform) laid out on its own; past the window's first, the barrier kept
             int tr = -1;
             plan_keys(ps, F, Dc, s_idx[j], s_flag[j]);
-            plan_in_tile(ps, g, F, ndr, Tcap, row_bytes, trash_row, j == 0 ? 0u : kMetaUnpaired, s_c,
+            plan_in_tile<NT>(ps, g, F, ndr, Tcap, row_bytes, trash_row, j == 0 ? 0u : kMetaUnpaired, s_c,
                          s_toff, tfeat, tsrc, meta, &tr);
             s_ftile[j][tid] = mine ? tr : -1;
             __syncthreads();
             continue;
         }
-        for (int rr = tid; rr < ndr; rr += 256) {
+        for (int rr = tid; rr < ndr; rr += NT) {
             int* m = meta + (g * ndr + rr) * kMetaStride;
             m[0] = s_toff[rr] | (s_toff[rr + 1] << 16);
             m[1] = s_toff[rr + 1];
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __
         }
         __syncthreads();
         const int nslots = s_toff[ndr] * 16;
-        for (int i = tid; i < nslots; i += 256) {
+        for (int i = tid; i < nslots; i += NT) {
             const int t = i / 16, p = i % 16;
             int rr = 0;
             while (t >= s_toff[rr + 1]) ++rr;
@@ -600,14 +603,25 @@ __global__ __launch_bounds__(256) void bwdf_plan_window_kernel(const int32_t* __
 // The plan of p: the staged build's in windows of groups, the others per group.
 void launch_plan(const int32_t* idx, int* tfeat, int* tsrc, int* perm, int* meta, int64_t F,
                  int64_t D, const BwdFPlan& p, hipStream_t st) {
-    if (p.staged)
-        bwdf_plan_window_kernel<<<dim3((unsigned)ceil_div(p.Gc, (int64_t)kPlanWindow)), dim3(256), 0, st>>>(
-            idx, tfeat, tsrc, perm, meta, (int)F, (int)D, (int)p.ndr, (int)p.Dc, (int)p.Tcap,
-            acc_stride((int)p.BT) * 4, (int)p.DCMAX, p.Gc);
+    // one thread per slot: the plan's time goes to its barriers and serial parts,
+    // which idle waves only lengthen (256 threads at O = 670,091, F = 64: about
+    // 240 us, 64 threads 104)
+    const dim3 windows((unsigned)ceil_div(p.Gc, (int64_t)kPlanWindow));
+#define HASTE_PLAN_WIN(NT)                                                                      \
+    bwdf_plan_window_kernel<NT><<<windows, dim3(NT), 0, st>>>(                                   \
+        idx, tfeat, tsrc, perm, meta, (int)F, (int)D, (int)p.ndr, (int)p.Dc, (int)p.Tcap,       \
+        acc_stride((int)p.BT) * 4, (int)p.DCMAX, p.Gc)
+    if (p.staged && F <= 64)
+        HASTE_PLAN_WIN(64);
+    else if (p.staged && F <= 128)
+        HASTE_PLAN_WIN(128);
+    else if (p.staged)
+        HASTE_PLAN_WIN(256);
     else
         bwdf_plan_kernel<<<dim3((unsigned)p.Gc), dim3(256), 0, st>>>(
             idx, tfeat, tsrc, perm, meta, (int)F, (int)D, (int)p.ndr, (int)p.Dc, (int)p.Tcap,
             acc_stride((int)p.BT) * 4, (int)p.DCMAX);
+#undef HASTE_PLAN_WIN
 }
 
 // ------------------------------------------------------------- gather ------

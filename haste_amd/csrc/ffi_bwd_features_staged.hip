@@ -12,8 +12,12 @@ template <typename T, int G, bool YA>
 int staged_bt(const int* tfeat, const int* meta, const uint16_t* twt, const uint16_t* dY,
               int64_t lddy, float* ws, const BwdFPlan& p, int64_t B, int64_t D, int64_t O,
               hipStream_t st) {
-    if (p.BT == 64) return launch_staged<T, G, 64, 8, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
-    return launch_staged<T, G, 32, 8, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
+    if (p.tiles < kStagedTiles) {
+        if (p.BT == 64) return launch_staged<T, G, 64, 8, 4, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
+        return launch_staged<T, G, 32, 8, 4, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
+    }
+    if (p.BT == 64) return launch_staged<T, G, 64, 8, 8, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
+    return launch_staged<T, G, 32, 8, 8, YA>(tfeat, meta, twt, dY, lddy, ws, p, B, D, O, st);
 }
 template <typename T, int G>
 int staged_ya(bool ya, const int* tfeat, const int* meta, const uint16_t* twt, const uint16_t* dY,
