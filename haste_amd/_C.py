@@ -83,6 +83,19 @@ def grad_rows(t: torch.Tensor) -> Tuple[torch.Tensor, int]:
     return rows_aligned(t)
 
 
+def compute_rows(t: torch.Tensor) -> Tuple[torch.Tensor, int]:
+    """grad_rows of grad_output as the kernels compute with it: fp32 rows are
+    rounded to fp16 into a buffer whose rows start on 128-byte lines."""
+    if t.dtype != torch.float32 or t.shape[0] >= 65536 or t.shape[1] < 2 or t.stride(1) != 1 \
+            or t.stride(0) < t.shape[1] or t.numel() == 0 or not t.is_cuda:
+        return grad_rows(f16_compute(t))
+    ld = round64(t.shape[1])
+    buf = torch.empty(t.shape[0], ld, dtype=torch.float16, device=t.device)
+    _lib.call("haste_cast_rows_f16", t.data_ptr(), t.stride(0), buf.data_ptr(), ld, t.shape[0],
+              t.shape[1], stream_of(t))
+    return buf[:, : t.shape[1]], ld
+
+
 def padded_transpose(features: torch.Tensor) -> Tuple[torch.Tensor, int]:
     """features [B, D] -> (xT [D, B] view of a [D, round8(B)] buffer, ld), by the
     HIP transpose kernel (padding columns are zero)."""
@@ -218,7 +231,7 @@ def ffi_backward_features_cuda(features: torch.Tensor, weights: torch.Tensor,
         raise RuntimeError(f"grad_outputs must be [B={B}, L={L}] (got {list(grad_outputs.shape)})")
     if grad_outputs.dtype != weights.dtype:
         raise RuntimeError("grad_outputs dtype must match weights dtype")
-    dY, lddy = grad_rows(f16_compute(grad_outputs))
+    dY, lddy = compute_rows(grad_outputs)
     W = f16_compute(weights).contiguous()
     ws = bwd_features_workspace(B, H, FANIN, L, gsize, W.dtype, weights.device)
     out = torch.empty(H, B, dtype=torch.float32, device=weights.device)

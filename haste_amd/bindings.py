@@ -131,7 +131,7 @@ def _ffi_grads(xT: torch.Tensor, weights: torch.Tensor, group_locations: torch.T
     # an fp32 layer computes with fp16 copies of W, X and grad_output, as the
     # reference's fp32 kernels round them when they load them
     f32 = dtype == torch.float32
-    dY, lddy = _C.grad_rows(_C.f16_compute(grad_output))
+    dY, lddy = _C.compute_rows(grad_output)
     locs = group_locations.contiguous()
     W = _C.f16_compute(weights).contiguous()
     stream = _C.stream_of(W)

@@ -5,7 +5,8 @@ Semantics kept from the reference:
   * per param group, ``seed`` is read and then incremented by 1 on every
     step (optim_sr.py:59-62); every tensor of the group uses that seed with
     offsets restarting at 0 (so weights and bias share random streams);
-  * fp32 params take the plain torch path (optim_sr.py:73-84);
+  * fp32 params take the plain update (optim_sr.py:73-84), contiguous ones on the
+    device as one fused kernel with the torch ops' roundings;
   * low-precision params are updated in place by one fused kernel (one
     launch per gradient dtype covers all of the group's tensors)
     (g' = fma(wd, w, g); m' = fma(mu, m, g'); w' = fma(-lr, m' or g', w);
@@ -167,17 +168,23 @@ class SRSgd(Optimizer):
             stepped = {id(b) for b in fused_bias.values()}
 
             # bf16 tensors are updated by one fused launch per gradient dtype
-            batches = {}
+            batches, f32s = {}, []
             for p in group["params"]:
                 if p.grad is None or id(p) in stepped:
                     continue
                 grad = p.grad
 
                 if p.dtype == torch.float32:
+                    buf = self._momentum_buf(p) if mom_on else None
+                    if (p.is_cuda and p.is_contiguous() and grad.dtype == torch.float32
+                            and grad.device == p.device and grad.layout == torch.strided
+                            and grad.is_contiguous() and grad.shape == p.shape
+                            and (buf is None or (buf.is_contiguous() and buf.shape == p.shape))):
+                        f32s.append((p, grad, buf))
+                        continue
                     if wd != 0.0:
                         grad = grad.add(p, alpha=wd)
                     if mom_on:
-                        buf = self._momentum_buf(p)
                         buf.mul_(mu).add_(grad)
                         update = buf
                     else:
@@ -221,6 +228,18 @@ class SRSgd(Optimizer):
                 b[1].append(g_contig)
                 b[2].append(self._momentum_buf(p) if mom_on else None)
                 b[3].append(p)
+            by_dev = {}
+            for t in f32s:
+                by_dev.setdefault(t[0].device, []).append(t)
+            for ts in by_dev.values():
+                arr = (_lib.SgdTensor * len(ts))(*[
+                    _lib.SgdTensor(p.data_ptr(), g.data_ptr(),
+                                   None if m is None else m.data_ptr(), p.numel(), 0)
+                    for p, g, m in ts])
+                _lib.call("haste_sgd_step_f32_multi", arr, len(ts), float(lr), float(wd), float(mu),
+                          int(mom_on), _C.stream_of(ts[0][0]))
+                for p, _, m in ts:
+                    torch.autograd.graph.increment_version(p if m is None else (p, m))
             for ws, gs, ms, ps in batches.values():
                 sgd_update_multi(ws, gs, ms if mom_on else None, learning_rate=lr,
                                  weight_decay=wd, momentum=mu, use_momentum=use_mom,

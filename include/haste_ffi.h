@@ -441,6 +441,25 @@ int haste_sgd_sr_step_multi(const haste_sgd_tensor* tensors, int32_t count, int3
                             uint64_t seed, void* stream);
 
 /*
+ * The SGD step of fp32 parameters (shared_ffi/optim_sr.py:73-84, torch ops in the
+ * reference), one launch per 8 tensors: tensor i's w, g and m are fp32 (offset0
+ * unused); g' = fma(wd, w, g) if wd != 0, m' = round(mu * m) + g' with use_mom,
+ * w' = fma(-lr, m' or g', w): the roundings of torch's add(alpha=) and mul.
+ */
+int haste_sgd_step_f32_multi(const haste_sgd_tensor* tensors, int32_t count, float lr, float wd,
+                             float mu, int32_t use_mom, void* stream);
+
+/*
+ * out[r, c] = fp16(in[r, c]) to nearest even, c < cols (columns up to the next
+ * multiple of 8: zero).  in fp32 at any row stride ldi >= cols, out 16-byte
+ * aligned with ldo a multiple of 8, rows < 65536: the fp16 grad_output of an
+ * fp32 layer (the reference's kernels round it as they load it,
+ * ffi_backward_features.cu:288-303) in rows that start on 16-byte boundaries.
+ */
+int haste_cast_rows_f16(const float* in, int64_t ldi, uint16_t* out, int64_t ldo, int64_t rows,
+                        int64_t cols, void* stream);
+
+/*
  * xT[d, b] = x[b, d] for a bf16/f16 matrix x [B, D] with row stride ldx;
  * xT has row stride ldt >= B, and columns B..ldt-1 of xT are set to zero.
  * Replaces features.transpose(0, 1).contiguous() (shared_ffi/bindings.py:19).
