@@ -138,9 +138,10 @@ def _ffi_grads(xT: torch.Tensor, weights: torch.Tensor, group_locations: torch.T
     code = _C.dtype_code(W.dtype)
 
     grad_x = None
-    # bf16 layer with weight or bias gradients too: dX is finished by the
-    # weight-gradient launch (haste_ffi_bwd_weights_dx) instead of a reduce kernel
-    dx_in_w = need_x and dtype == torch.bfloat16 and (need_w or need_b)
+    # with weight or bias gradients too, dX is finished by the weight-gradient
+    # launch (haste_ffi_bwd_weights_dx[_rne]) instead of kernels of its own (an
+    # fp32 layer's bias gradient is not that launch's)
+    dx_in_w = need_x and (need_w or (need_b and not f32))
     if need_x:
         ent = _bwdf_workspace(locs, B, D, F, O, gsize, W.dtype, stream)
         ws = ent.ws
@@ -187,7 +188,13 @@ def _ffi_grads(xT: torch.Tensor, weights: torch.Tensor, group_locations: torch.T
         else:  # bias only: the kernel still needs a dW target
             scratch = torch.empty(O, F, dtype=W.dtype, device=dev)
             dw_ptr, dw_code = scratch.data_ptr(), code
-        if dx_in_w:
+        if dx_in_w and dtype != torch.bfloat16:
+            _lib.call("haste_ffi_bwd_weights_dx_rne", locs.data_ptr(), xT.data_ptr(), ldx,
+                      dY.data_ptr(), lddy, dw_ptr, dw_code, grad_b.data_ptr() if need_b else None,
+                      _C.dtype_code(bias_dtype) if need_b else 0, grad_x.data_ptr(),
+                      _C.dtype_code(dtype), ws.data_ptr(), ws.numel(), B, D, F, O, gsize, code,
+                      stream)
+        elif dx_in_w:
             _lib.call("haste_ffi_bwd_weights_dx", locs.data_ptr(), xT.data_ptr(), ldx,
                       dY.data_ptr(), lddy, dw_ptr, dw_code, grad_b.data_ptr() if need_b else None,
                       _C.dtype_code(bias_dtype) if need_b else 0, grad_x.data_ptr(),

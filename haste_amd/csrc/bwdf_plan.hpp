@@ -147,18 +147,19 @@ __device__ __forceinline__ f32x4 sum_slices(const float* __restrict__ ws, int64_
 // The final pass of backward to features with stochastic rounding, as a job of
 // ntiles tiles of 32 features x 32 batch columns (nx tiles along D): sum the
 // slices, transpose [D, B] -> [B, D] and round to bf16 with
-// tl.randint(seed, b*D + d).
+// tl.randint(seed, b*D + d); or (out_dtype) to fp16 to nearest even, or fp32.
 struct ReduceJob {
     const float* ws;
-    uint16_t* dX;
+    void* dX;
     int B, Bp, D, S, nx, ntiles;
     uint32_t k0, k1;
+    int out_dtype;  // HASTE_DTYPE_BF16 (0, stochastic), _F16 or _F32
 };
 
-inline ReduceJob reduce_job(const BwdFPlan& p, const float* ws, uint16_t* dX, int64_t B,
-                            int64_t D, uint64_t seed) {
+inline ReduceJob reduce_job(const BwdFPlan& p, const float* ws, void* dX, int64_t B, int64_t D,
+                            uint64_t seed, int out_dtype = HASTE_DTYPE_BF16) {
     ReduceJob j{ws, dX, (int)B, (int)p.Bp, (int)D, (int)p.S, (int)ceil_div(D, 32), 0,
-                (uint32_t)seed, (uint32_t)(seed >> 32)};
+                (uint32_t)seed, (uint32_t)(seed >> 32), out_dtype};
     j.ntiles = j.nx * (int)ceil_div(B, 32);
     return j;
 }
@@ -179,8 +180,13 @@ __device__ __forceinline__ void reduce_sr_tile(const ReduceJob& j, int tile, flo
         const int b = b0 + r, d = d0 + tx;
         if (d < j.D && b < j.B) {
             const uint64_t off = (uint64_t)b * j.D + d;
-            j.dX[(int64_t)b * j.D + d] = (uint16_t)sr_bf16(
-                t[tx][r], philox_w0((uint32_t)off, (uint32_t)(off >> 32), 0u, j.k0, j.k1));
+            if (j.out_dtype == HASTE_DTYPE_F32)
+                static_cast<float*>(j.dX)[off] = t[tx][r];
+            else if (j.out_dtype == HASTE_DTYPE_F16)
+                static_cast<uint16_t*>(j.dX)[off] = (uint16_t)f32_to_f16_rne(t[tx][r]);
+            else
+                static_cast<uint16_t*>(j.dX)[off] = (uint16_t)sr_bf16(
+                    t[tx][r], philox_w0((uint32_t)off, (uint32_t)(off >> 32), 0u, j.k0, j.k1));
         }
     }
 }

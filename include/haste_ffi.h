@@ -245,6 +245,19 @@ int haste_ffi_bwd_weights_dx(const int32_t* idx, const void* xT, int64_t ldx, co
                              void* stream);
 
 /*
+ * The same for an fp16 layer (dX_dtype fp16: the sums rounded to nearest even) and
+ * for an fp32 layer on fp16 copies (dX_dtype fp32: the sums): what
+ * haste_ffi_bwd_features's dX^T transposed and converted gives, bit for bit
+ * (shared_ffi/bindings.py:44-50).
+ */
+int haste_ffi_bwd_weights_dx_rne(const int32_t* idx, const void* xT, int64_t ldx, const void* dY,
+                                 int64_t lddy, void* dW, int32_t dW_dtype, void* dbias,
+                                 int32_t dbias_dtype, void* dX, int32_t dX_dtype,
+                                 void* bwdf_workspace, int64_t bwdf_workspace_bytes, int64_t B,
+                                 int64_t D, int64_t F, int64_t O, int64_t G, int32_t dtype,
+                                 void* stream);
+
+/*
  * Backward to weights fused with the SR-SGD step on the bf16 weights and bias:
  * computes the fp32 gradients of haste_ffi_bwd_weights and applies to W [O, F]
  * and bias [O] (in place) the update of haste_sgd_sr_step with g = those fp32
