@@ -88,6 +88,15 @@ SIGNATURES = {
                                                             _I32, _U64, _P, _P, _U64, _P, _I64,
                                                             _I64, _I64, _I64, _I64, _I64, _I32,
                                                             _P]),
+    "haste_transpose_features_labels": (ctypes.c_int, [_P, _I64, _P, _I64, _I64, _I64, _P, _I64,
+                                                       _P, _I64, _I64, _I64, _P]),
+    "haste_ffi_forward_bce_marked": (ctypes.c_int, [_P, _P, _I64, _P, _P, _P, _I64, _P, _I64, _I64,
+                                                    _I64, _I64, _I64, _I64, _I32, _P]),
+    "haste_ffi_bwd_weights_sgd_dx_loss": (ctypes.c_int, [_P, _P, _I64, _P, _I64, _P, _P, _P, _P,
+                                                         _F32, _F32, _F32, _I32, _I32, _U64, _P,
+                                                         _P, _U64, _P, _I64, _P, _I64, _P, _P,
+                                                         _I64, _I64, _I64, _I64, _I64, _I64, _I32,
+                                                         _P]),
     "haste_sgd_sr_step_wt": (ctypes.c_int, [_P, _P, _I32, _P, _F32, _F32, _F32, _I32, _I32, _U64,
                                             _P, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P]),
     "haste_sgd_sr_step_wt_bias": (ctypes.c_int, [_P, _P, _I32, _P, _P, _P, _I32, _P, _F32, _F32,

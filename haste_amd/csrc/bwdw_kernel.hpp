@@ -44,6 +44,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "bce_job.hpp"
 #include "bwdf_plan.hpp"
 
 namespace haste {
@@ -71,6 +72,7 @@ struct SgdArgs {
     const uint64_t* seed_dev;  // not NULL: the Philox seed is read here (k0, k1 unused)
     uint16_t* logits;  // FWD launches: the logits [B, ldl]
     int64_t ldl;
+    BceJob lj;  // lj.nblk > 0: workgroups after rj's sum this loss
 };
 
 namespace {
@@ -182,7 +184,11 @@ __global__ __launch_bounds__(kThreads, (bwdw_waves_per_simd<G, FP, FWD>())) void
     // more than the others, and it is then that one
     const int64_t Gc = (O + G - 1) / G;
     if (blockIdx.x >= Gc) {  // the reduce job's tiles (sg.rj.ntiles > 0)
-        reduce_sr_tile(sg.rj, (int)(blockIdx.x - Gc), reinterpret_cast<float (*)[33]>(lds));
+        const int64_t b = blockIdx.x - Gc;
+        if (b < sg.rj.ntiles)
+            reduce_sr_tile(sg.rj, (int)b, reinterpret_cast<float (*)[33]>(lds));
+        else
+            sum_loss(sg.lj, b - sg.rj.ntiles, reinterpret_cast<float*>(lds));
         return;
     }
     const int64_t g = blockIdx.x == 0 ? Gc - 1 : (int64_t)blockIdx.x - 1;
@@ -666,13 +672,13 @@ int launch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16_t* 
            void* dW, int dW_dtype, void* dbias, int dbias_dtype, int64_t B, int64_t D, int64_t F,
            int64_t O, const SgdArgs& sg, hipStream_t st) {
     const int64_t Gc = ceil_div(O, G);
-    if (Gc + sg.rj.ntiles > 0x7FFFFFFF || D * ldx * 2 > kMaxRsrcBytes ||
+    if (Gc + sg.rj.ntiles + sg.lj.nblk > 0x7FFFFFFF || D * ldx * 2 > kMaxRsrcBytes ||
         ((int64_t)BwdWCfg<G, FP, FWD>::KC * lddy + 8) * 2 > kMaxRsrcBytes || (int64_t)G * F * 4 > kMaxRsrcBytes) {
         set_error("haste_ffi_bwd_weights: problem too large (Gc %lld, lddy %lld, D*ldx %lld)",
                   (long long)Gc, (long long)lddy, (long long)(D * ldx));
         return HASTE_ERR_UNSUPPORTED;
     }
-    ffi_bwd_w_kernel<T, G, FP, SGD, YNT, YS, FWD><<<dim3((unsigned)(Gc + sg.rj.ntiles)), dim3(kThreads), 0, st>>>(
+    ffi_bwd_w_kernel<T, G, FP, SGD, YNT, YS, FWD><<<dim3((unsigned)(Gc + sg.rj.ntiles + sg.lj.nblk)), dim3(kThreads), 0, st>>>(
         idx, xT, ldx, dY, lddy, dW, dW_dtype, dbias, dbias_dtype, (int)B, (int)D, (int)F, O, sg);
     HASTE_CHECK_LAUNCH("haste_ffi_bwd_weights");
     return HASTE_OK;

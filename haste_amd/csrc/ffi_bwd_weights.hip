@@ -149,7 +149,8 @@ int bwdw_sgd(const char* fn, const int32_t* idx, const void* xT, int64_t ldx, co
              int32_t use_mom, int32_t do_sr, uint64_t seed, uint16_t* dX, uint64_t dx_seed,
              void* bwdf_workspace, int64_t bwdf_workspace_bytes, int64_t B, int64_t D, int64_t F,
              int64_t O, int64_t G, int32_t dtype, void* stream,
-             const uint64_t* seed_dev = nullptr, uint16_t* logits = nullptr, int64_t ldl = 0) {
+             const uint64_t* seed_dev = nullptr, uint16_t* logits = nullptr, int64_t ldl = 0,
+             const BceJob& lj = BceJob{}) {
     int rc = check_bwdw(fn, idx, xT, ldx, dY, lddy, dW_dtype, dbias, dbias_dtype, B, D, F, O, G,
                         dtype);
     if (rc != HASTE_OK) return rc;
@@ -165,7 +166,7 @@ int bwdw_sgd(const char* fn, const int32_t* idx, const void* xT, int64_t ldx, co
                     "%s: momentum buffers missing or misaligned", fn);
     SgdArgs sg{W, bias, m_W, m_bias, lr, wd, mu, use_mom ? 1 : 0, do_sr ? 1 : 0,
                (uint32_t)seed, (uint32_t)(seed >> 32), nullptr, nullptr, nullptr, nullptr,
-               0, 0, ReduceJob{}, seed_dev, logits, ldl};
+               0, 0, ReduceJob{}, seed_dev, logits, ldl, lj};
     if (bwdf_workspace != nullptr) {
         const BwdFPlan p = make_plan(B, D, F, O, G);
         HASTE_CHECK_ARG(aligned16(bwdf_workspace) &&
@@ -280,6 +281,31 @@ extern "C" int haste_ffi_forward_bwd_weights_sgd_dx(
                              HASTE_DTYPE_F32, nullptr, HASTE_DTYPE_F32, lr, wd, mu, use_mom,
                              do_sr, seed, dX, dx_seed, bwdf_workspace, bwdf_workspace_bytes, B, D,
                              F, O, G, dtype, stream, seed_dev, logits, ldl);
+    if (rc != HASTE_OK || seed_dev == nullptr) return rc;
+    haste::seed_advance_kernel<<<dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream)>>>(seed_dev);
+    HASTE_CHECK_LAUNCH(fn);
+    return HASTE_OK;
+}
+
+extern "C" int haste_ffi_bwd_weights_sgd_dx_loss(
+    const int32_t* idx, const void* xT, int64_t ldx, const void* dY, int64_t lddy, uint16_t* W,
+    uint16_t* bias, float* m_W, float* m_bias, float lr, float wd, float mu, int32_t use_mom,
+    int32_t do_sr, uint64_t seed, uint64_t* seed_dev, uint16_t* dX, uint64_t dx_seed,
+    void* bwdf_workspace, int64_t bwdf_workspace_bytes, const int32_t* labels, int64_t nnz,
+    float* loss, void* bce_workspace, int64_t bce_ws_bytes, int64_t B, int64_t D, int64_t F,
+    int64_t O, int64_t G, int32_t dtype, void* stream) {
+    const char* fn = "haste_ffi_bwd_weights_sgd_dx_loss";
+    HASTE_CHECK_ARG(dX != nullptr && bwdf_workspace != nullptr && loss != nullptr,
+                    "%s: dX, the bwd-features workspace and loss are required", fn);
+    HASTE_CHECK_ARG(seed_dev == nullptr || reinterpret_cast<uintptr_t>(seed_dev) % 8 == 0,
+                    "%s: seed_dev must be 8-byte aligned", fn);
+    int rc = haste::check_bce_job(fn, labels, nnz, bce_workspace, bce_ws_bytes, B, O, G);
+    if (rc != HASTE_OK) return rc;
+    rc = haste::bwdw_sgd(fn, idx, xT, ldx, dY, lddy, W, bias, m_W, m_bias, nullptr, HASTE_DTYPE_F32,
+                         nullptr, HASTE_DTYPE_F32, lr, wd, mu, use_mom, do_sr, seed, dX, dx_seed,
+                         bwdf_workspace, bwdf_workspace_bytes, B, D, F, O, G, dtype, stream,
+                         seed_dev, nullptr, 0,
+                         haste::bce_job(labels, nnz, bce_workspace, loss, B, O, G));
     if (rc != HASTE_OK || seed_dev == nullptr) return rc;
     haste::seed_advance_kernel<<<dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream)>>>(seed_dev);
     HASTE_CHECK_LAUNCH(fn);

@@ -28,7 +28,7 @@
 #include <algorithm>
 #include <mutex>
 
-#include "common.hpp"
+#include "bce_job.hpp"
 
 namespace haste {
 namespace {
@@ -540,51 +540,12 @@ int dispatch_g(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16
     return HASTE_ERR_UNSUPPORTED;
 }
 
-// Label bits of the COO positives (row, label) pairs, ored into the (all zero)
-// bitmap; loss_sum_kernel clears the words again after the forward.  Pairs
-// outside [0, B) x [0, O) are ignored.
-__global__ __launch_bounds__(256) void label_bits_kernel(const int32_t* __restrict__ labels,
-                                                         int64_t nnz, uint32_t* __restrict__ ybits,
-                                                         int64_t ldyw, int B, int64_t O) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nnz) return;
-    const int r = labels[2 * i], c = labels[2 * i + 1];
-    if (r < 0 || r >= B || c < 0 || c >= O) return;
-    atomicOr(ybits + (int64_t)r * ldyw + c / 32, 1u << (c % 32));
+__global__ __launch_bounds__(256) void label_bits_kernel(const BceJob j) {
+    mark_labels(j, blockIdx.x);
 }
-
-// loss = sum of the n workgroup partials (workgroup 0): each thread sums a
-// strided subset in order, then a fixed tree over the threads.  Every
-// workgroup also clears the label words of 256 of the call's pairs (one launch
-// instead of two small ones).
-__global__ __launch_bounds__(256) void loss_sum_kernel(const float* __restrict__ part, int64_t n,
-                                                       float* __restrict__ loss,
-                                                       const int32_t* __restrict__ labels,
-                                                       int64_t nnz, uint32_t* __restrict__ ybits,
-                                                       int64_t ldyw, int B, int64_t O) {
+__global__ __launch_bounds__(256) void loss_sum_kernel(const BceJob j) {
     __shared__ float s[256];
-    const int64_t li = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (li < nnz) {
-        const int r = labels[2 * li], c = labels[2 * li + 1];
-        if (r >= 0 && r < B && c >= 0 && c < O) ybits[(int64_t)r * ldyw + c / 32] = 0u;
-    }
-    if (blockIdx.x != 0) return;
-    // the partials in batches of 8 loads in flight, summed in index order
-    float v = 0.0f;
-    for (int64_t i0 = threadIdx.x; i0 < n; i0 += 8 * 256) {
-        float pv[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) pv[k] = i0 + k * 256 < n ? part[i0 + k * 256] : 0.0f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v += pv[k];
-    }
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int m = 128; m >= 1; m >>= 1) {
-        if ((int)threadIdx.x < m) s[threadIdx.x] += s[threadIdx.x + m];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *loss = s[0];
+    sum_loss(j, blockIdx.x, s);
 }
 
 struct BceLayout {
@@ -602,6 +563,25 @@ BceLayout bce_layout(int64_t B, int64_t O, int64_t G) {
 }
 
 }  // namespace
+
+BceJob bce_job(const int32_t* labels, int64_t nnz, void* workspace, float* loss, int64_t B,
+               int64_t O, int64_t G) {
+    const BceLayout L = bce_layout(B, O, G);
+    return BceJob{labels, nnz, static_cast<uint32_t*>(workspace), L.ldyw, (int)B, O,
+                  reinterpret_cast<const float*>(static_cast<char*>(workspace) + L.bits_bytes),
+                  L.nparts, loss, (int)std::max<int64_t>(1, ceil_div(nnz, 256))};
+}
+
+int check_bce_job(const char* fn, const int32_t* labels, int64_t nnz, const void* workspace,
+                  int64_t ws_bytes, int64_t B, int64_t O, int64_t G) {
+    HASTE_CHECK_ARG(nnz >= 0 && (labels || nnz == 0) && nnz < (int64_t)1 << 31,
+                    "%s: null labels or invalid nnz", fn);
+    const int64_t need = haste_ffi_forward_bce_workspace_size(B, O, G);
+    HASTE_CHECK_ARG(need >= 0 && workspace != nullptr && aligned16(workspace) && ws_bytes >= need,
+                    "%s: workspace missing, misaligned or too small (%lld < %lld bytes)", fn,
+                    (long long)ws_bytes, (long long)need);
+    return HASTE_OK;
+}
 
 // Shape checks shared by the three FFI entry points.
 int check_ffi_shape(const char* fn, int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
@@ -692,31 +672,38 @@ extern "C" int64_t haste_ffi_forward_bce_workspace_size(int64_t B, int64_t O, in
 namespace haste {
 namespace {
 
+// The forward with the BCE epilogue, on a checked workspace whose label bits are set.
+int run_forward_marked(const int32_t* idx, const void* xT, int64_t ldx, const void* W,
+                       const void* bias, void* dY, int64_t ldo, void* logits, void* workspace,
+                       const BceLayout& L, int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
+                       int32_t dtype, hipStream_t st) {
+    auto* ybits = static_cast<uint32_t*>(workspace);
+    float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + L.bits_bytes);
+    const BceArgs bce{ybits, L.ldyw, static_cast<uint16_t*>(logits), part};
+    auto* x = static_cast<const uint16_t*>(xT);
+    auto* w = static_cast<const uint16_t*>(W);
+    auto* bb = static_cast<const uint16_t*>(bias);
+    auto* o = static_cast<uint16_t*>(dY);
+    return dtype == HASTE_DTYPE_BF16
+               ? dispatch_g<BF16>(idx, x, ldx, w, bb, o, ldo, B, D, F, O, G, &bce, st)
+               : dispatch_g<F16>(idx, x, ldx, w, bb, o, ldo, B, D, F, O, G, &bce, st);
+}
+
 // Launches of haste_ffi_forward_bce on a checked workspace: label bits, the
 // forward with the BCE epilogue, the loss sum (which clears the label bits).
 int run_forward_bce(const int32_t* idx, const void* xT, int64_t ldx, const void* W,
                     const void* bias, const int32_t* labels, int64_t nnz, void* dY, int64_t ldo,
                     void* logits, float* loss, void* workspace, const BceLayout& L, int64_t B,
                     int64_t D, int64_t F, int64_t O, int64_t G, int32_t dtype, hipStream_t st) {
-    auto* ybits = static_cast<uint32_t*>(workspace);
-    float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + L.bits_bytes);
-    const int64_t lblocks = (nnz + 255) / 256;
-    if (lblocks > 0) {
-        label_bits_kernel<<<dim3((unsigned)lblocks), dim3(256), 0, st>>>(labels, nnz, ybits,
-                                                                          L.ldyw, (int)B, O);
+    const BceJob job = bce_job(labels, nnz, workspace, loss, B, O, G);
+    if (nnz > 0) {
+        label_bits_kernel<<<dim3((unsigned)job.nblk), dim3(256), 0, st>>>(job);
         HASTE_CHECK_LAUNCH("haste_ffi_forward_bce");
     }
-    const BceArgs bce{ybits, L.ldyw, static_cast<uint16_t*>(logits), part};
-    auto* x = static_cast<const uint16_t*>(xT);
-    auto* w = static_cast<const uint16_t*>(W);
-    auto* bb = static_cast<const uint16_t*>(bias);
-    auto* o = static_cast<uint16_t*>(dY);
-    int rc = dtype == HASTE_DTYPE_BF16
-                 ? dispatch_g<BF16>(idx, x, ldx, w, bb, o, ldo, B, D, F, O, G, &bce, st)
-                 : dispatch_g<F16>(idx, x, ldx, w, bb, o, ldo, B, D, F, O, G, &bce, st);
+    int rc = run_forward_marked(idx, xT, ldx, W, bias, dY, ldo, logits, workspace, L, B, D, F, O, G,
+                                dtype, st);
     if (rc != HASTE_OK) return rc;
-    loss_sum_kernel<<<dim3((unsigned)std::max<int64_t>(1, ceil_div(nnz, 256))), dim3(256), 0, st>>>(
-        part, L.nparts, loss, labels, nnz, ybits, L.ldyw, (int)B, O);
+    loss_sum_kernel<<<dim3((unsigned)job.nblk), dim3(256), 0, st>>>(job);
     HASTE_CHECK_LAUNCH("haste_ffi_forward_bce");
     return HASTE_OK;
 }
@@ -848,4 +835,21 @@ extern "C" int haste_ffi_forward_bce_noalloc(const int32_t* idx, const void* xT,
     HASTE_CHECK_LAUNCH(fn);
     return haste::run_forward_bce(idx, xT, ldx, W, bias, labels, nnz, dY, ldo, logits, loss, ws,
                                   L, B, D, F, O, G, dtype, st);
+}
+
+extern "C" int haste_ffi_forward_bce_marked(const int32_t* idx, const void* xT, int64_t ldx,
+                                            const void* W, const void* bias, void* dY,
+                                            int64_t ldo, void* workspace, int64_t ws_bytes,
+                                            int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
+                                            int32_t dtype, void* stream) {
+    const char* fn = "haste_ffi_forward_bce_marked";
+    float unused = 0.0f;
+    int rc = haste::check_forward_bce(fn, idx, xT, ldx, W, nullptr, 0, dY, ldo, nullptr, &unused, B,
+                                      D, F, O, G, dtype);
+    if (rc != HASTE_OK) return rc;
+    rc = haste::check_bce_job(fn, nullptr, 0, workspace, ws_bytes, B, O, G);
+    if (rc != HASTE_OK) return rc;
+    return haste::run_forward_marked(idx, xT, ldx, W, bias, dY, ldo, nullptr, workspace,
+                                     haste::bce_layout(B, O, G), B, D, F, O, G, dtype,
+                                     static_cast<hipStream_t>(stream));
 }

@@ -133,13 +133,8 @@ class FFITrainStep:
                   self.code, _C.stream_of(self.W))
         return self.logits
 
-    def forward_bce(self, x: torch.Tensor, labels: torch.Tensor,
-                    write_logits: bool = False) -> torch.Tensor:
-        """Forward fused with the sparse BCE loss (src/runner.py:469-478): ``labels``
-        is the COO [nnz, 2] int32 (row, label) list of positives.  Writes
-        dY = sigma(logits) - Y into ``dY_buf`` ([B, ldo]; the logits into
-        ``logits_buf`` too when ``write_logits``) and returns the summed loss as a
-        0-d fp32 tensor (computed on the device, no host sync)."""
+    def _bce_inputs(self, x: torch.Tensor, labels: torch.Tensor):
+        """x and labels checked and contiguous, the BCE buffers allocated."""
         if tuple(x.shape) != (self.B, self.D) or x.dtype != torch.bfloat16:
             raise ValueError(f"FFITrainStep.forward_bce: x must be bf16 [{self.B}, {self.D}] "
                              f"(got {x.dtype} {list(x.shape)})")
@@ -157,6 +152,16 @@ class FFITrainStep:
             self.bce_ws = torch.zeros(n, dtype=torch.uint8, device=self.W.device)
             self.dY_buf = torch.zeros(self.B, self.ldo, dtype=torch.bfloat16, device=self.W.device)
             self.loss_buf = torch.zeros((), dtype=torch.float32, device=self.W.device)
+        return x, labels
+
+    def forward_bce(self, x: torch.Tensor, labels: torch.Tensor,
+                    write_logits: bool = False) -> torch.Tensor:
+        """Forward fused with the sparse BCE loss (src/runner.py:469-478): ``labels``
+        is the COO [nnz, 2] int32 (row, label) list of positives.  Writes
+        dY = sigma(logits) - Y into ``dY_buf`` ([B, ldo]; the logits into
+        ``logits_buf`` too when ``write_logits``) and returns the summed loss as a
+        0-d fp32 tensor (computed on the device, no host sync)."""
+        x, labels = self._bce_inputs(x, labels)
         st = _C.stream_of(self.W)
         _lib.call("haste_transpose_features", x.data_ptr(), x.stride(0), self.xT_buf.data_ptr(),
                   self.ldx, self.B, self.D, st)
@@ -172,10 +177,41 @@ class FFITrainStep:
         """A training step with the loss fused into the forward: forward + BCE
         gradient -> backward to features (dX) -> fused weight/bias gradient +
         SR-SGD.  Returns the loss (0-d fp32 device tensor) of the step's forward."""
-        loss = self.forward_bce(x, labels)
-        self.backward_features(self.dY_buf, self.ldo, defer_dx=True)
-        self.backward_weights_sgd(self.dY_buf, self.ldo)
-        return loss
+        if self.grad_dtype != torch.float32 or labels.numel() > 1 << 21:
+            loss = self.forward_bce(x, labels)
+            self.backward_features(self.dY_buf, self.ldo, defer_dx=True)
+            self.backward_weights_sgd(self.dY_buf, self.ldo)
+            return loss
+        # forward_bce's label and loss kernels ride in the transpose's and the
+        # update's launches (bit-identical to the calls above; up to 2^20 pairs,
+        # which those grids have room for)
+        x, labels = self._bce_inputs(x, labels)
+        st = _C.stream_of(self.W)
+        bias = None if self.bias is None else self.bias.data_ptr()
+        try:
+            _lib.call("haste_transpose_features_labels", x.data_ptr(), x.stride(0),
+                      self.xT_buf.data_ptr(), self.ldx, self.B, self.D, labels.data_ptr(),
+                      labels.shape[0], self.bce_ws.data_ptr(), self.bce_ws.numel(), self.O, self.G,
+                      st)
+            _lib.call("haste_ffi_forward_bce_marked", self.idx.data_ptr(), self.xT_buf.data_ptr(),
+                      self.ldx, self.W.data_ptr(), bias, self.dY_buf.data_ptr(), self.ldo,
+                      self.bce_ws.data_ptr(), self.bce_ws.numel(), self.B, self.D, self.F, self.O,
+                      self.G, self.code, st)
+            self.backward_features(self.dY_buf, self.ldo, defer_dx=True)
+            seed_dev = None if self._seed_dev is None else self._seed_dev.data_ptr()
+            _lib.call("haste_ffi_bwd_weights_sgd_dx_loss", self.idx.data_ptr(),
+                      self.xT_buf.data_ptr(), self.ldx, self.dY_buf.data_ptr(), self.ldo,
+                      self.W.data_ptr(), bias, None, None, self.lr, self.wd, 0.0, 0, 1, self.seed,
+                      seed_dev, self.dX.data_ptr(), SR_SEED_GRAD_X, self.ws.data_ptr(),
+                      self.ws.numel(), labels.data_ptr(), labels.shape[0],
+                      self.loss_buf.data_ptr(), self.bce_ws.data_ptr(), self.bce_ws.numel(),
+                      self.B, self.D, self.F, self.O, self.G, self.code, st)
+        except BaseException:
+            self.bce_ws.zero_()  # the label bits of a step broken off
+            raise
+        self._dx_pending = False
+        self._weights_updated(True)
+        return self.loss_buf
 
     def _check_dY(self, dY: torch.Tensor, lddy: int) -> None:
         _C.require_device(dY, "dY")

@@ -356,6 +356,35 @@ int haste_ffi_forward_bwd_weights_sgd_dx(
     int64_t F, int64_t O, int64_t G, int32_t dtype, void* stream);
 
 /*
+ * haste_ffi_forward_bce as part of a training step, its small kernels run as extra
+ * workgroups of launches that the step makes anyway, in this order on one stream:
+ *   haste_transpose_features_labels: haste_transpose_features, and the label bits
+ *     set in the BCE workspace;
+ *   haste_ffi_forward_bce_marked: dY and the loss partials from those bits;
+ *   (haste_ffi_bwd_features_partials)
+ *   haste_ffi_bwd_weights_sgd_dx_loss: haste_ffi_bwd_weights_sgd_dx (seed_dev not
+ *     NULL: ..._dev_seed), and the loss, the bits of the same labels cleared.
+ * The workspace must be zero before the first; the last leaves it zero (a step
+ * broken off between them must clear it).  Bit-identical to haste_ffi_forward_bce
+ * and the separate calls.
+ */
+int haste_transpose_features_labels(const uint16_t* x, int64_t ldx, uint16_t* xT, int64_t ldt,
+                                    int64_t B, int64_t D, const int32_t* labels, int64_t nnz,
+                                    void* bce_workspace, int64_t bce_ws_bytes, int64_t O,
+                                    int64_t G, void* stream);
+int haste_ffi_forward_bce_marked(const int32_t* idx, const void* xT, int64_t ldx, const void* W,
+                                 const void* bias, void* dY, int64_t ldo, void* workspace,
+                                 int64_t ws_bytes, int64_t B, int64_t D, int64_t F, int64_t O,
+                                 int64_t G, int32_t dtype, void* stream);
+int haste_ffi_bwd_weights_sgd_dx_loss(
+    const int32_t* idx, const void* xT, int64_t ldx, const void* dY, int64_t lddy, uint16_t* W,
+    uint16_t* bias, float* m_W, float* m_bias, float lr, float wd, float mu, int32_t use_mom,
+    int32_t do_sr, uint64_t seed, uint64_t* seed_dev, uint16_t* dX, uint64_t dx_seed,
+    void* bwdf_workspace, int64_t bwdf_workspace_bytes, const int32_t* labels, int64_t nnz,
+    float* loss, void* bce_workspace, int64_t bce_ws_bytes, int64_t B, int64_t D, int64_t F,
+    int64_t O, int64_t G, int32_t dtype, void* stream);
+
+/*
  * haste_sgd_sr_step_wt that also steps the layer's bias [O] (bf16) with its
  * gradient gb [O] (bf16, f16 or f32) and fp32 momentum m_bias (read and written
  * when use_mom), in the same launch: the same update as haste_sgd_sr_step on
