@@ -14,7 +14,8 @@ step time then stays flat for seconds), then exactly K timed steps.  Inputs are
 synthetic and resident in HBM before timing; the grad of the logits
 dY = bf16(sigmoid(z) - Y) is computed once from the initial logits (BASELINE
 configs: Y binary, ~5 positives per row (10 at config 4), Zipf(1.1) over
-labels).  "hip_graph" is the same step captured once in a HIP graph and
+labels).  "hip_graph" is the same step as one FFITrainStep.step call, whose
+update launch also computes the logits, captured once in a HIP graph and
 replayed (the SR-SGD seed is read and advanced on the device).  "fused_loss"
 times the step a training loop runs instead: the
 forward computes dY = sigma(z) - Y and the BCE loss from the COO labels in its
