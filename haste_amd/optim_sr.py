@@ -6,7 +6,8 @@ Semantics kept from the reference:
     step (optim_sr.py:59-62); every tensor of the group uses that seed with
     offsets restarting at 0 (so weights and bias share random streams);
   * fp32 params take the plain update (optim_sr.py:73-84), contiguous ones on the
-    device as one fused kernel with the torch ops' roundings;
+    current device as one fused kernel with the torch ops' roundings, any others
+    by those ops;
   * low-precision params are updated in place by one fused kernel (one
     launch per gradient dtype covers all of the group's tensors)
     (g' = fma(wd, w, g); m' = fma(mu, m, g'); w' = fma(-lr, m' or g', w);
@@ -42,6 +43,64 @@ from . import bindings as _bindings
 from .sr import sgd_update_multi
 
 __all__ = ["SRSgd", "SGD_SR"]
+
+
+def _fusable_f32(p, grad, buf, device) -> bool:
+    """Whether the kernel, which gets addresses only, may step the fp32 parameter p:
+    plain tensors (a subclass may keep its values elsewhere) on ``device``, the one
+    its launch runs on, contiguous fp32 of one shape.  A momentum buffer can differ:
+    it is created with the optimizer, before its model may move."""
+    return all(type(t) is torch.Tensor and t.device == device and t.dtype == torch.float32
+               and t.layout == torch.strided and t.shape == p.shape and t.is_contiguous()
+               and not t.is_neg()
+               for t in ((p.data, grad) if buf is None else (p.data, grad, buf)))
+
+
+def _overlapping(f32s) -> bool:
+    """Whether memory that the step of one of the (parameter, grad, momentum)
+    triples writes is used by another's: their steps then depend on their order."""
+    spans = []
+    for p, grad, buf in f32s:
+        for t, written in ((p.data, True), (grad, False), (buf, True)):
+            if type(t) is torch.Tensor and t.layout == torch.strided and t.numel():
+                n = 1 + sum((s - 1) * st for s, st in zip(t.shape, t.stride()))
+                spans.append((t.data_ptr(), t.data_ptr() + n * t.element_size(), written))
+    spans.sort()
+    end = end_written = 0
+    for lo, hi, written in spans:
+        if lo < end_written or (written and lo < end):
+            return True
+        end = max(end, hi)
+        if written:
+            end_written = max(end_written, hi)
+    return False
+
+
+def _step_f32(f32s, lr, wd, mu, mom_on) -> None:
+    """Step the fp32 (parameter, grad, momentum or None) triples of a group."""
+    fused = []
+    if any(p.is_cuda for p, _, _ in f32s) and not _overlapping(f32s):
+        device = torch.device("cuda", torch.cuda.current_device())
+        fused = [t for t in f32s if _fusable_f32(*t, device)]
+    keep = {id(p) for p, _, _ in fused}
+    for p, grad, buf in f32s:
+        if id(p) in keep:
+            continue
+        if wd != 0.0:
+            grad = grad.add(p, alpha=wd)
+        if mom_on:
+            buf.mul_(mu).add_(grad)
+            grad = buf
+        p.add_(grad, alpha=-lr)
+    if not fused:
+        return
+    arr = (_lib.SgdTensor * len(fused))(*[
+        _lib.SgdTensor(p.data_ptr(), g.data_ptr(), None if m is None else m.data_ptr(),
+                       p.numel(), 0) for p, g, m in fused])
+    _lib.call("haste_sgd_step_f32_multi", arr, len(fused), float(lr), float(wd), float(mu),
+              int(mom_on), _C.stream_of(fused[0][0]))
+    for p, _, m in fused:
+        torch.autograd.graph.increment_version(p if m is None else (p, m))
 
 
 class SRSgd(Optimizer):
@@ -175,21 +234,7 @@ class SRSgd(Optimizer):
                 grad = p.grad
 
                 if p.dtype == torch.float32:
-                    buf = self._momentum_buf(p) if mom_on else None
-                    if (p.is_cuda and p.is_contiguous() and grad.dtype == torch.float32
-                            and grad.device == p.device and grad.layout == torch.strided
-                            and grad.is_contiguous() and grad.shape == p.shape
-                            and (buf is None or (buf.is_contiguous() and buf.shape == p.shape))):
-                        f32s.append((p, grad, buf))
-                        continue
-                    if wd != 0.0:
-                        grad = grad.add(p, alpha=wd)
-                    if mom_on:
-                        buf.mul_(mu).add_(grad)
-                        update = buf
-                    else:
-                        update = grad
-                    p.add_(update, alpha=-lr)
+                    f32s.append((p, grad, self._momentum_buf(p) if mom_on else None))
                     continue
 
                 w = p.data
@@ -228,18 +273,8 @@ class SRSgd(Optimizer):
                 b[1].append(g_contig)
                 b[2].append(self._momentum_buf(p) if mom_on else None)
                 b[3].append(p)
-            by_dev = {}
-            for t in f32s:
-                by_dev.setdefault(t[0].device, []).append(t)
-            for ts in by_dev.values():
-                arr = (_lib.SgdTensor * len(ts))(*[
-                    _lib.SgdTensor(p.data_ptr(), g.data_ptr(),
-                                   None if m is None else m.data_ptr(), p.numel(), 0)
-                    for p, g, m in ts])
-                _lib.call("haste_sgd_step_f32_multi", arr, len(ts), float(lr), float(wd), float(mu),
-                          int(mom_on), _C.stream_of(ts[0][0]))
-                for p, _, m in ts:
-                    torch.autograd.graph.increment_version(p if m is None else (p, m))
+            if f32s:
+                _step_f32(f32s, lr, wd, mu, mom_on)
             for ws, gs, ms, ps in batches.values():
                 sgd_update_multi(ws, gs, ms if mom_on else None, learning_rate=lr,
                                  weight_decay=wd, momentum=mu, use_momentum=use_mom,
