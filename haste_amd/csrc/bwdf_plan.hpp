@@ -92,23 +92,29 @@ inline double ring_overflow(int64_t F, double q, int rt) {
     return s + std::exp(lp);  // n = F
 }
 
-// The smallest ring whose rounds overflow for under 1 % of (group, range)
-// pairs.  Plans are made on every call, so the last shape's choice is kept
-// (per host thread) instead of summing the binomial tail again.
+// Whether more than 1 % of (group, range) pairs overflow rt tiles.  Plans are made
+// on every call and the sum takes 2 - 6 us, so the answers are kept, in a table
+// per host thread that the shapes of a program's layers share.
+inline bool overflows(int64_t F, double q, int rt) {
+    struct Entry {
+        double q;
+        int64_t F;
+        int rt;
+        bool yes;
+    };
+    thread_local Entry table[64] = {};  // F = 0: empty
+    Entry& e = table[((F / 16) * 4 + rt + (int64_t)(q * 4096.0) * 7) & 63];
+    if (e.F != F || e.q != q || e.rt != rt) e = Entry{q, F, rt, ring_overflow(F, q, rt) >= 0.01};
+    return e.yes;
+}
+
+// The smallest ring whose rounds overflow for under 1 % of (group, range) pairs.
 inline int64_t pick_ring(int64_t BT, int64_t D, int64_t F, int64_t G) {
-    thread_local int64_t key[4] = {-1, -1, -1, -1};
-    thread_local int64_t last = 0;
-    if (key[0] == BT && key[1] == D && key[2] == F && key[3] == G) return last;
-    int64_t ring = ring_tiles((int)G);
+    const int64_t ring = ring_tiles((int)G);
     for (int rt = 2; rt <= 3 && rt < ring; ++rt) {
         const int64_t dc = ceil_div(D, ceil_div(D, (int64_t)max_dc((int)BT, (int)G, rt)));
-        if (ring_overflow(F, std::min(1.0, (double)dc / (double)D), rt) < 0.01) {
-            ring = rt;
-            break;
-        }
+        if (!overflows(F, std::min(1.0, (double)dc / (double)D), rt)) return rt;
     }
-    key[0] = BT; key[1] = D; key[2] = F; key[3] = G;
-    last = ring;
     return ring;
 }
 
@@ -250,7 +256,7 @@ inline BwdFPlan make_plan_for(int64_t B, int64_t D, int64_t F, int64_t O, int64_
     p.ndr = ceil_div(D, p.DCMAX);
     p.tiles = kStagedTiles;
     if (p.staged && F > (p.ndr == 1 ? 48 : 32 * p.ndr) &&
-        ring_overflow(F, 1.0 / (double)p.ndr, kStagedTiles / 2) < 0.01)
+        !overflows(F, 1.0 / (double)p.ndr, kStagedTiles / 2))
         p.tiles = kStagedTiles / 2;
     p.Dc = ceil_div(D, p.ndr);
     int64_t S = std::max<int64_t>(1, kTargetCTAs / (p.nbt * p.ndr));

@@ -237,6 +237,30 @@ def test_staged_cases_reach_every_staged_build():
     assert kernel_config(L, 100, 300, 1000, 16, 16)[1] > 0        # G = 16: ring
 
 
+def test_plans_of_alternating_layers_cost_no_tail_sums():
+    """The bwd-features plan, made on every call, keeps its binomial tail sums: for
+    the shapes of three layers in turn it takes about the time of one without any."""
+    import time
+
+    L = _lib.lib()
+    cfg = (ctypes.c_int64 * 4)()
+    f = L.haste_ffi_bwd_features_config
+
+    def best(shapes):
+        t = []
+        for _ in range(100):
+            t0 = time.perf_counter()
+            for _ in range(20):
+                for s in shapes:
+                    f(*s, 0, cfg)
+            t.append((time.perf_counter() - t0) / (20 * len(shapes)))
+        return min(t)
+
+    plain = best([(37, 768, 64, 2000, 64)])  # one range of four tiles: no sum
+    layers = [(37, 1500, 256, 2000, 64), (256, 2500, 128, 9000, 32), (256, 3000, 256, 9000, 32)]
+    assert best(layers) < 2 * plain + 5e-7
+
+
 def test_sr_words_fold_rejects_bad_arguments():
     L = _lib.lib()
     assert L.haste_sr_words_fold(None, -1, 0, None) == _lib.HASTE_ERR_INVALID_ARG
