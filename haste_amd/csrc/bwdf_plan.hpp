@@ -280,26 +280,44 @@ inline BwdFPlan make_plan_for(int64_t B, int64_t D, int64_t F, int64_t O, int64_
     return p;
 }
 
+// Whether the staged plan p with two waves to a tile is faster than the other
+// builds' plan r.  Measured over some 2,500 shapes with B = 1 .. 1024, O = 3,000 ..
+// 670,091, D up to 4,500 and one to seven ranges (time of p / time of r, geometric
+// mean, extremes):
+//  - B <= 32: 0.63 (0.37 - 0.93);
+//  - fewer than 3/4 of r's workgroups (batches of 1024, whose units leave one
+//    slice): 1.07 (0.96 - 1.26) at G = 64 and 128, so r;
+//  - G = 64 and 128 otherwise: 0.74 (0.41 - 1.12) and 0.65 (0.29 - 1.15);
+//  - G = 32, whose products are one MFMA deep, so that what a group costs beside
+//    them counts: one range where r needs several, 0.70 (0.51 - 0.97; the fp32 layer
+//    at O = 131,073, F = 64, B = 256, D = 768: 104 -> 51 us), ranges that r covers in two
+//    tiles, 0.79 (0.55 - 1.03), or in three with the same batch tile, 0.71 (0.59 - 0.85);
+//  - G = 32 otherwise: 1.00 (0.52 - 1.48), above 1 for most of them, so r.
+inline bool half_pays(const BwdFPlan& p, const BwdFPlan& r, int64_t B, int64_t G) {
+    if (B <= 32) return true;
+    if (4 * p.nbt * p.ndr * p.S < 3 * r.nbt * r.ndr * r.S) return false;
+    if (G > 32) return true;
+    return p.ndr == 1 ? r.ndr > 1 : r.RT == 2 || (r.RT == 3 && r.BT == p.BT);
+}
+
 // The plan of the build that haste_ffi_bwd_features_set_build selects (1 ring,
 // 2 direct, 3 staged; 0: by shape).  By shape, G >= 32 takes the staged build
 // where a group's range holds seven or more tiles of 16 positions, so that
 // nearly all of its eight waves have a tile (measured, config 1: 86 -> 82 us;
 // config 4: 3452 -> 2402 us; with four tiles, configs 2 and 3, it was slower
-// than the ring and direct builds: 295 -> 336 and 606 -> 805 us).  With two
-// waves to a tile it is the faster one for ranges of at most four tiles, too,
-// measured: 345 -> 300 us at O = 670,091, G = F = 64, B = 512, D = 768; 185 -> 157
-// (two ranges: G = 64, F = 96, D = 1500, O = 300,000, B = 256); 212 -> 202 (G = 32,
-// F = 80, D = 1700); 104 -> 51 (fp32 layer, G = 32, F = 64, B = 256, O = 131,073);
-// three tiles in one range (F = 48) were slower: 202 -> 206.  Either way the slice's
-// W^T tiles must span at most kMaxRsrcBytes (its 32-bit tile offsets).
+// than the ring and direct builds: 295 -> 336 and 606 -> 805 us), and with two
+// waves to a tile for ranges of at most four tiles where half_pays (345 -> 300 us
+// at O = 670,091, G = F = 64, B = 512, D = 768; three tiles in one range, F = 48, were
+// slower: 202 -> 206).  Either way the slice's W^T tiles must span at most
+// kMaxRsrcBytes (its 32-bit tile offsets).
 inline BwdFPlan make_plan(int64_t B, int64_t D, int64_t F, int64_t O, int64_t G) {
     const int build = bwdf_build();
-    if (G >= 32 && (build == 0 || build == 3)) {
-        const BwdFPlan p = make_plan_for(B, D, F, O, G, true);
-        const bool fits = (p.gps + 8) * p.Tcap * 16 * G * 2 <= kMaxRsrcBytes;
-        if (fits && (build == 3 || F >= 7 * 16 * p.ndr || p.tiles < kStagedTiles)) return p;
-    }
-    return make_plan_for(B, D, F, O, G, false);
+    if (G < 32 || (build != 0 && build != 3)) return make_plan_for(B, D, F, O, G, false);
+    const BwdFPlan p = make_plan_for(B, D, F, O, G, true);
+    const bool fits = (p.gps + 8) * p.Tcap * 16 * G * 2 <= kMaxRsrcBytes;
+    if (fits && (build == 3 || F >= 7 * 16 * p.ndr)) return p;
+    const BwdFPlan r = make_plan_for(B, D, F, O, G, false);
+    return fits && p.tiles < kStagedTiles && half_pays(p, r, B, G) ? p : r;
 }
 
 // One 16-byte chunk (labels lc .. lc+7 of the group) of the W^T row described by

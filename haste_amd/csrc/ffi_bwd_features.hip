@@ -956,6 +956,14 @@ extern "C" int haste_ffi_bwd_features_config(int64_t B, int64_t D, int64_t F, in
     return HASTE_OK;
 }
 
+extern "C" int64_t haste_ffi_bwd_features_tiles(int64_t B, int64_t D, int64_t F, int64_t O,
+                                                int64_t G, int32_t dtype) {
+    int rc = haste::check_ffi_shape("haste_ffi_bwd_features_tiles", B, D, F, O, G, dtype);
+    if (rc != HASTE_OK) return rc;
+    const haste::BwdFPlan p = haste::make_plan(B, D, F, O, G);
+    return p.staged ? p.tiles : 0;
+}
+
 namespace haste {
 static std::atomic<int> g_bwdf_build{0};
 int bwdf_build() { return g_bwdf_build.load(std::memory_order_relaxed); }

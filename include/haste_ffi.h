@@ -147,8 +147,16 @@ int haste_ffi_bwd_features_config(int64_t B, int64_t D, int64_t F, int64_t O, in
                                   int32_t dtype, int64_t* cfg);
 
 /*
+ * The tiles that the staged build keeps in its pipeline for these sizes: 8 with a
+ * wave to a tile, 4 with two; 0 where another build runs.  Host-only, negative
+ * HASTE_ERR_* codes as above.
+ */
+int64_t haste_ffi_bwd_features_tiles(int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
+                                     int32_t dtype);
+
+/*
  * Selects the main kernel of later bwd-features calls in this process
- * (host-only): 0 (the default) and 3 the staged build for G >= 32, else the
+ * (host-only): 0 (the default) by shape; 3 the staged build for G >= 32, else the
  * LDS-ring build; 1 always the LDS-ring build; 2 the direct build wherever it
  * exists (G = 32 or 64, and a group slice's transposed weights under 2 GB),
  * else the ring build.  The builds give the same

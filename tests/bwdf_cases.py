@@ -9,7 +9,9 @@ chosen per shape by the library's plan.  RING_CASES holds one shape per build
 The staged build (the default for G >= 32, set_build(3)) is compiled per
 (G, BT) with G in {32, 64, 128} and BT in {32, 64}.  STAGED_CASES holds one
 shape per (G, BT, more than one feature range); G = 128 takes 64 batch columns
-only where the whole of D fits one range.
+only where the whole of D fits one range.  Ranges of at most four tiles of 16 have
+builds of their own with two waves to a tile: HALF_CASES, one shape per (G, BT,
+more than one range), and up to seven ranges.
 
 tests/test_abi.py checks on the CPU that the library maps the cases onto
 every build, tests/test_gpu_ffi.py runs them against the oracle.
@@ -46,6 +48,14 @@ STAGED_CASES = [
     (37, 300, 2000, 64, 16, "random"), (37, 1000, 2000, 64, 16, "dups"),
     (37, 768, 2000, 128, 16, "random"), (37, 1500, 2000, 128, 16, "dups"),
     (37, 200, 2000, 128, 16, "dups"),
+]
+
+
+HALF_CASES = [
+    (37, 600, 2000, 32, 64), (40, 1600, 2000, 32, 80), (37, 200, 2000, 32, 64),
+    (100, 1100, 1999, 32, 112), (33, 3200, 2001, 32, 240), (37, 500, 2000, 64, 64),
+    (97, 2900, 2000, 64, 144), (37, 100, 2000, 64, 64), (37, 2000, 1993, 64, 176),
+    (1, 300, 2000, 128, 64), (33, 4000, 2000, 128, 208), (40, 200, 2000, 128, 64),
 ]
 
 

@@ -237,6 +237,36 @@ def test_staged_cases_reach_every_staged_build():
     assert kernel_config(L, 100, 300, 1000, 16, 16)[1] > 0        # G = 16: ring
 
 
+def test_half_cases_reach_every_build_with_two_waves_to_a_tile():
+    from bwdf_cases import HALF_CASES, kernel_config, staged_variants
+
+    L = _lib.lib()
+    seen, ranges = set(), set()
+    prev = L.haste_ffi_bwd_features_set_build(3)
+    try:
+        for B, D, O, G, F in HALF_CASES:
+            assert L.haste_ffi_bwd_features_tiles(B, D, F, O, G, 0) == 4, (B, D, O, G, F)
+            BT, _RT, ndr, _S = kernel_config(L, B, D, O, G, F)
+            seen.add((G, BT, ndr >= 2))
+            ranges.add(ndr)
+    finally:
+        L.haste_ffi_bwd_features_set_build(prev)
+    assert seen == staged_variants() and {1, 2, 4, 5, 6, 7} <= ranges
+
+
+@pytest.mark.parametrize("tiles,B,D,O,G,F", [
+    # measured faster: one and several ranges, small batches at any size, G = 32 where the
+    # other builds split further
+    (4, 512, 768, 670091, 64, 64), (4, 256, 768, 131073, 32, 64), (4, 16, 298, 3000, 32, 64),
+    (4, 32, 4000, 20011, 128, 208), (4, 256, 1500, 300000, 64, 96),
+    # measured slower: 43 -> 64 us, 102 -> 132, 186 -> 275, 46 -> 58 (one slice)
+    (0, 512, 201, 131073, 32, 64), (0, 256, 2090, 131073, 32, 176), (0, 400, 3321, 131073, 32, 144),
+    (0, 1024, 4061, 10007, 64, 192),
+])
+def test_two_waves_to_a_tile_where_it_is_faster(tiles, B, D, O, G, F):
+    assert _lib.lib().haste_ffi_bwd_features_tiles(B, D, F, O, G, 0) == tiles
+
+
 def test_plans_of_alternating_layers_cost_no_tail_sums():
     """The bwd-features plan, made on every call, keeps its binomial tail sums: for
     the shapes of three layers in turn it takes about the time of one without any."""

@@ -4,7 +4,8 @@ import pytest
 import torch
 
 import oracle
-from haste_amd import _C
+from bwdf_cases import HALF_CASES
+from haste_amd import _C, _lib
 from test_gpu_ffi import TOL32, make_case
 
 pytestmark = pytest.mark.gpu
@@ -24,5 +25,20 @@ def test_two_waves_to_a_tile(dev, B, D, O, G, F, mode):
     idx[-2] = torch.arange(F, dtype=torch.int32)
     dXT = _C.ffi_backward_features_cuda(x.t().contiguous().to(dev), W.to(dev), idx.to(dev),
                                         dY.to(dev), B, D, F, O, G)
+    ref = oracle.ffi_backward_features(idx, W, dY, G, D)
+    torch.testing.assert_close(dXT.cpu(), ref, **TOL32)
+
+
+@pytest.mark.parametrize("mode", ["random", "dups"])
+@pytest.mark.parametrize("B,D,O,G,F", HALF_CASES)
+def test_every_build_with_two_waves_to_a_tile(dev, B, D, O, G, F, mode):
+    """One shape per build (tests/test_abi.py checks the coverage), whatever the default is."""
+    x, W, bias, idx, dY = make_case(B, D, O, G, F, idx_mode=mode, seed=D)
+    prev = _lib.lib().haste_ffi_bwd_features_set_build(3)
+    try:
+        dXT = _C.ffi_backward_features_cuda(x.t().contiguous().to(dev), W.to(dev), idx.to(dev),
+                                            dY.to(dev), B, D, F, O, G)
+    finally:
+        _lib.lib().haste_ffi_bwd_features_set_build(prev)
     ref = oracle.ffi_backward_features(idx, W, dY, G, D)
     torch.testing.assert_close(dXT.cpu(), ref, **TOL32)
