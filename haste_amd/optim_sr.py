@@ -50,24 +50,29 @@ def _fusable_f32(p, grad, buf, device) -> bool:
     plain tensors (a subclass may keep its values elsewhere) on ``device``, the one
     its launch runs on, contiguous fp32 of one shape.  A momentum buffer can differ:
     it is created with the optimizer, before its model may move."""
-    return all(type(t) is torch.Tensor and t.device == device and t.dtype == torch.float32
-               and t.layout == torch.strided and t.shape == p.shape and t.is_contiguous()
-               and not t.is_neg()
-               for t in ((p.data, grad) if buf is None else (p.data, grad, buf)))
+    shape = p.shape
+    for t in (p.data, grad) if buf is None else (p.data, grad, buf):
+        if not (type(t) is torch.Tensor and t.dtype is torch.float32 and t.device == device
+                and t.layout is torch.strided and t.is_contiguous() and t.shape == shape
+                and not t.is_neg()):
+            return False
+    return True
 
 
-def _overlapping(f32s) -> bool:
-    """Whether memory that the step of one of the (parameter, grad, momentum)
-    triples writes is used by another's: their steps then depend on their order."""
-    spans = []
-    for p, grad, buf in f32s:
-        for t, written in ((p.data, True), (grad, False), (buf, True)):
-            if type(t) is torch.Tensor and t.layout == torch.strided and t.numel():
-                n = 1 + sum((s - 1) * st for s, st in zip(t.shape, t.stride()))
-                spans.append((t.data_ptr(), t.data_ptr() + n * t.element_size(), written))
-    spans.sort()
+def _span(t):
+    """[first, last) byte of t's memory; None for tensors without such a range."""
+    if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.layout is not torch.strided \
+            or t.numel() == 0:
+        return None
+    n = 1 + sum((s - 1) * st for s, st in zip(t.shape, t.stride()))
+    return t.data_ptr(), t.data_ptr() + n * t.element_size()
+
+
+def _overlapping(spans) -> bool:
+    """Whether memory that the step of one tensor writes is used by another's (their
+    steps then depend on their order), from (first, last, written) ranges."""
     end = end_written = 0
-    for lo, hi, written in spans:
+    for lo, hi, written in sorted(spans):
         if lo < end_written or (written and lo < end):
             return True
         end = max(end, hi)
@@ -77,15 +82,30 @@ def _overlapping(f32s) -> bool:
 
 
 def _step_f32(f32s, lr, wd, mu, mom_on) -> None:
-    """Step the fp32 (parameter, grad, momentum or None) triples of a group."""
-    fused = []
-    if any(p.is_cuda for p, _, _ in f32s) and not _overlapping(f32s):
-        device = torch.device("cuda", torch.cuda.current_device())
-        fused = [t for t in f32s if _fusable_f32(*t, device)]
-    keep = {id(p) for p, _, _ in fused}
+    """Step the fp32 (parameter, grad, momentum or None) triples of a group: by the
+    kernel those it may step by address, the others by torch's ops in their order,
+    as all of them where their memory overlaps."""
+    fused, others, spans = [], [], []
+    device = None
     for p, grad, buf in f32s:
-        if id(p) in keep:
-            continue
+        if device is None and p.is_cuda:
+            device = torch.device("cuda", torch.cuda.current_device())
+        if device is not None and _fusable_f32(p, grad, buf, device):
+            n = p.numel()
+            t = (p.data_ptr(), grad.data_ptr(), None if buf is None else buf.data_ptr(), n, 0)
+            fused.append(t)
+            if n:
+                spans += [(t[0], t[0] + 4 * n, True), (t[1], t[1] + 4 * n, False)]
+                if buf is not None:
+                    spans.append((t[2], t[2] + 4 * n, True))
+        else:
+            others.append((p, grad, buf))
+    if fused and others:
+        spans += [(*s, t is not g) for p, g, m in others for t in (p, g, m)
+                  if t is not None and (s := _span(t)) is not None]
+    if fused and _overlapping(spans):
+        fused, others = [], f32s
+    for p, grad, buf in others:
         if wd != 0.0:
             grad = grad.add(p, alpha=wd)
         if mom_on:
@@ -94,13 +114,13 @@ def _step_f32(f32s, lr, wd, mu, mom_on) -> None:
         p.add_(grad, alpha=-lr)
     if not fused:
         return
-    arr = (_lib.SgdTensor * len(fused))(*[
-        _lib.SgdTensor(p.data_ptr(), g.data_ptr(), None if m is None else m.data_ptr(),
-                       p.numel(), 0) for p, g, m in fused])
+    arr = (_lib.SgdTensor * len(fused))(*fused)
     _lib.call("haste_sgd_step_f32_multi", arr, len(fused), float(lr), float(wd), float(mu),
-              int(mom_on), _C.stream_of(fused[0][0]))
-    for p, _, m in fused:
-        torch.autograd.graph.increment_version(p if m is None else (p, m))
+              int(mom_on), torch._C._cuda_getCurrentRawStream(device.index))
+    if others:
+        f32s = [t for t in f32s if all(t[0] is not o[0] for o in others)]
+    torch.autograd.graph.increment_version(
+        [t for p, _, m in f32s for t in ((p,) if m is None else (p, m))])
 
 
 class SRSgd(Optimizer):

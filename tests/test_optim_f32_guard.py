@@ -42,18 +42,23 @@ def test_any_other_parameter(data):
     assert not optim_sr._fusable_f32(p, torch.ones(6), None, CPU)
 
 
+def overlapping(triples):
+    return optim_sr._overlapping([(*optim_sr._span(t), t is not g) for p, g, m in triples
+                                  for t in (p, g, m) if t is not None and optim_sr._span(t)])
+
+
 def test_overlapping():
     flat = torch.zeros(12)
     a, b, c = (torch.nn.Parameter(flat[i:j]) for i, j in ((0, 6), (6, 12), (5, 7)))
     g, h = torch.ones(6), torch.ones(2)
-    assert not optim_sr._overlapping([(a, g, None), (b, g, None)])   # a shared grad is only read
-    assert optim_sr._overlapping([(a, g, None), (c, h, None)])
-    assert optim_sr._overlapping([(a, g, None), (a, g, None)])
-    assert optim_sr._overlapping([(a, b.data, None), (b, g, None)])  # one's grad is the other
-    assert optim_sr._overlapping([(a, g, torch.zeros(6)), (b, g, flat[:6])])
+    assert not overlapping([(a, g, None), (b, g, None)])   # a shared grad is only read
+    assert overlapping([(a, g, None), (c, h, None)])
+    assert overlapping([(a, g, None), (a, g, None)])
+    assert overlapping([(a, b.data, None), (b, g, None)])            # one's grad is the other
+    assert overlapping([(a, g, torch.zeros(6)), (b, g, flat[:6])])
     t = torch.nn.Parameter(flat.view(3, 4).t())
-    assert optim_sr._overlapping([(b, g, None), (t, torch.ones(4, 3), None)])
-    assert not optim_sr._overlapping([(torch.nn.Parameter(torch.zeros(0)), torch.zeros(0), None)])
+    assert overlapping([(b, g, None), (t, torch.ones(4, 3), None)])
+    assert not overlapping([(torch.nn.Parameter(torch.zeros(0)), torch.zeros(0), None)])
 
 
 @pytest.mark.gpu
@@ -84,3 +89,23 @@ def test_shared_storage_is_stepped_in_order(dev, momentum):
             r.add_(u, alpha=-0.1)
         opt.step()
     assert torch.equal(w, ref)
+
+
+@pytest.mark.gpu
+def test_kernel_and_torch_ops_in_one_group(dev):
+    """Parameters for the kernel and one that is not contiguous, apart and sharing memory."""
+    for shared in (False, True):
+        w = torch.randn(40, 30, device=dev)
+        ts = [torch.randn(7, device=dev), w.t() if shared else torch.randn(30, 40, device=dev).t(),
+              w, torch.zeros(0, device=dev)]
+        ref = [t.clone() for t in ts]
+        if shared:
+            ref[1] = ref[2].t()
+        ps = [torch.nn.Parameter(t) for t in ts]
+        v = [p._version for p in ps]
+        for p, r in zip(ps, ref):
+            p.grad = torch.randn(p.shape, device=dev)
+            r.add_(p.grad, alpha=-0.5)
+        SRSgd(ps, lr=0.5).step()
+        assert all(torch.equal(p, r) for p, r in zip(ps, ref))
+        assert all(p._version > a for p, a in zip(ps, v))
