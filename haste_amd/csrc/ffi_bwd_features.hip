@@ -94,7 +94,7 @@ __device__ __forceinline__ void dup_free_slot(int k, int T0, int T1, int nd, int
 // = (tb | tm << 16, te): layer-0 tiles [tb, tm), layer-1 tiles [tm, te) (relative
 // to g*Tcap); meta[(g*ndr + ndr-1)*2 + 1] is the group's tile count.  The
 // staged build's plan is made in the in-tile mode instead (plan_in_tile,
-// bwdf_plan_pair_kernel): no layer 1 (tm = te); a duplicated feature's "lo"
+// bwdf_plan_window_kernel): no layer 1 (tm = te); a duplicated feature's "lo"
 // row sits in the same tile as its "hi" row, one position after it, and its
 // tfeat entry carries bit 0 (row offsets are multiples of 16).  For tile row
 // (t, p): tfeat = byte offset of the feature's row in the main kernel's LDS
@@ -226,7 +226,9 @@ __global__ __launch_bounds__(256) void bwdf_plan_kernel(const int32_t* __restric
 // holds), the group is laid out on its own and bit 31 of its meta word 0
 // (every range) tells the kernel to keep the barrier before its update.
 constexpr int kPairRanges = 8;     // ranges the pinned layout handles (else: unpaired)
-constexpr int kPairRangeTiles = 24;  // tiles of a range it tracks
+// Tiles of a range it tracks: twice the pipeline's four of a plan with two waves to
+// a tile, whose ranges hold no more in 99 % of groups; 24 else.
+__host__ __device__ constexpr int pair_range_tiles(bool half) { return half ? 8 : 24; }
 
 // One slot of a group's index row, as the plan sees it (thread tid = slot).
 struct PlanSlot {
@@ -234,56 +236,68 @@ struct PlanSlot {
     bool first;
 };
 
-// The analysis of group g's index row by the workgroup's threads: the
-// clamped indices in s_idx (padded to a multiple of 4 slots), first-occurrence /
-// duplicated flags in s_flag, perm, the per-range counts of distinct (s_c[0])
-// and duplicated (s_c[1]) features, and the thread's slot (pn / pd left 0, see
-// plan_keys).  s_c must be zero on entry.
-__device__ __forceinline__ PlanSlot plan_analyse(const int32_t* __restrict__ idx, int64_t g, int F,
-                                                 int D, int Dc, int* s_idx, int* s_flag,
-                                                 int (*s_c)[kMaxRanges], int* __restrict__ perm) {
+// The analysis of the index rows of groups g0 .. g0 + W - 1 (those below Gc) by the
+// workgroup's threads, thread = slot, the rows scanned together: the clamped
+// indices in s_idx (padded to a multiple of 4 slots), first-occurrence /
+// duplicated flags in s_flag, perm, the per-range counts of distinct (s_c[j][0])
+// and duplicated (s_c[j][1]) features, and the thread's slots (pn / pd left 0,
+// see plan_keys).  s_c must be zeroed before the first barrier here.
+template <int W, int NT>
+__device__ __forceinline__ void plan_analyse(const int32_t* __restrict__ idx, int64_t g0, int64_t Gc,
+                                             int F, int D, int Dc, int (*s_idx)[NT],
+                                             int (*s_flag)[NT], int (*s_c)[2][kMaxRanges],
+                                             int* __restrict__ perm, PlanSlot (&ps)[W]) {
     const int tid = threadIdx.x;
     const int F4 = (F + 3) & ~3;  // the rows are scanned 4 slots per 16-byte read
-    PlanSlot ps{0, 0, 0, 0, 0, 0, 0, false};
-    if (tid < F) s_idx[tid] = min(max(idx[g * F + tid], 0), D - 1);
-    else if (tid < F4) s_idx[tid] = INT_MAX;  // padding: matches and precedes no index
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        ps[j] = PlanSlot{0, 0, 0, 0, 0, 0, 0, false};
+        if (tid < F) s_idx[j][tid] = g0 + j < Gc ? min(max(idx[(g0 + j) * F + tid], 0), D - 1) : -1;
+        else if (tid < F4) s_idx[j][tid] = INT_MAX;  // padding: matches and precedes no index
+        if (tid < F4) s_flag[j][tid] = 0;
+    }
     __syncthreads();
-    const int4* idx4 = reinterpret_cast<const int4*>(s_idx);
     if (tid < F) {
-        ps.f = s_idx[tid];
-        int before = 0;
-#pragma unroll 4
+        int before[W] = {};
+#pragma unroll
+        for (int j = 0; j < W; ++j) ps[j].f = s_idx[j][tid];
+#pragma unroll 2
         for (int k4 = 0; k4 < F4 / 4; ++k4) {
-            const int4 v = idx4[k4];
             const int k = 4 * k4;
-            ps.rank += (v.x < ps.f) + (v.y < ps.f) + (v.z < ps.f) + (v.w < ps.f);
-            before += ((v.x == ps.f) & (k < tid)) + ((v.y == ps.f) & (k + 1 < tid)) +
-                      ((v.z == ps.f) & (k + 2 < tid)) + ((v.w == ps.f) & (k + 3 < tid));
-            ps.cnt += (v.x == ps.f) + (v.y == ps.f) + (v.z == ps.f) + (v.w == ps.f);
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const int4 v = reinterpret_cast<const int4*>(s_idx[j])[k4];
+                PlanSlot& q = ps[j];
+                q.rank += (v.x < q.f) + (v.y < q.f) + (v.z < q.f) + (v.w < q.f);
+                before[j] += ((v.x == q.f) & (k < tid)) + ((v.y == q.f) & (k + 1 < tid)) +
+                             ((v.z == q.f) & (k + 2 < tid)) + ((v.w == q.f) & (k + 3 < tid));
+                q.cnt += (v.x == q.f) + (v.y == q.f) + (v.z == q.f) + (v.w == q.f);
+            }
         }
-        ps.rank += before;
-        ps.first = before == 0;
-        perm[g * F + ps.rank] = tid;
-        s_flag[tid] = (ps.first ? 1 : 0) | (ps.cnt > 1 ? 2 : 0);
-    } else if (tid < F4) {
-        s_flag[tid] = 0;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            if (g0 + j >= Gc) continue;
+            PlanSlot& q = ps[j];
+            q.rank += before[j];
+            q.first = before[j] == 0;
+            perm[(g0 + j) * F + q.rank] = tid;
+            s_flag[j][tid] = (q.first ? 1 : 0) | (q.cnt > 1 ? 2 : 0);
+            q.r = q.f / Dc;
+            q.r_lo = q.r * Dc;
+            if (q.first) {
+                atomicAdd(&s_c[j][0][q.r], 1);
+                if (q.cnt > 1) atomicAdd(&s_c[j][1][q.r], 1);
+            }
+        }
     }
     __syncthreads();
-    ps.r = ps.f / Dc;
-    ps.r_lo = ps.r * Dc;
-    if (tid < F && ps.first) {
-        atomicAdd(&s_c[0][ps.r], 1);
-        if (ps.cnt > 1) atomicAdd(&s_c[1][ps.r], 1);
-    }
-    __syncthreads();
-    return ps;
 }
 
 // ps.pn / ps.pd of a first occurrence (the single / duplicated features of its
 // range with a smaller residue key), which plan_in_tile places by.
 __device__ __forceinline__ void plan_keys(PlanSlot& ps, int F, int Dc, const int* s_idx,
                                           const int* s_flag) {
-    if (!(threadIdx.x < F && ps.first)) return;
+    if (!ps.first) return;
     const int F4 = (F + 3) & ~3;
     const int key = (((ps.f - ps.r_lo) & 15) << 16) | (ps.f - ps.r_lo);
     const int4* idx4 = reinterpret_cast<const int4*>(s_idx);
@@ -304,33 +318,28 @@ __device__ __forceinline__ void plan_keys(PlanSlot& ps, int F, int Dc, const int
     }
 }
 
-// The in-tile layout of one group on its own (the staged build's plan): tiles per
-// range, meta (tm = te, bit 31 of word 0 = flag), the rows of the thread's
-// feature and the padding rows.  *t_rel receives the tile of the thread's
-// feature relative to its range's first.
+// The in-tile layout of one group on its own (the staged build's plan): meta (tm = te, bit 31 of word 0 = flag),
+// the rows of the thread's feature and the padding rows, from the tile offsets
+// of the ranges in s_toff.  Returns the tile of the thread's
+// feature relative to its range's first, or -1.
+__device__ __forceinline__ int range_tiles(const int (*s_c)[kMaxRanges], int r) {
+    return (s_c[0][r] + s_c[1][r] + 15) / 16;
+}
 template <int NT>
-__device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int F, int ndr, int Tcap,
-                                             int row_bytes, int trash_row, uint32_t flag,
-                                             int (*s_c)[kMaxRanges], int* s_toff,
-                                             int* __restrict__ tfeat, int* __restrict__ tsrc,
-                                             int* __restrict__ meta, int* t_rel) {
+__device__ __forceinline__ int plan_in_tile(const PlanSlot& ps, int64_t g, int ndr, int Tcap,
+                                            int row_bytes, int trash_row, uint32_t flag,
+                                            const int (*s_c)[kMaxRanges], const int* s_toff,
+                                            int* __restrict__ tfeat, int* __restrict__ tsrc,
+                                            int* __restrict__ meta) {
     const int tid = threadIdx.x;
-    if (tid == 0) {
-        int t = 0;
-        for (int rr = 0; rr < ndr; ++rr) {
-            s_toff[rr] = t;
-            t += (s_c[0][rr] + s_c[1][rr] + 15) / 16;
-        }
-        s_toff[ndr] = t;
-    }
-    __syncthreads();
+    int t_rel = -1;
     for (int rr = tid; rr < ndr; rr += NT) {
         int* m = meta + (g * ndr + rr) * kMetaStride;
         m[0] = (int)((uint32_t)s_toff[rr] | ((uint32_t)s_toff[rr + 1] << 16) | flag);
         m[1] = s_toff[rr + 1];
     }
     const int64_t tbase = g * Tcap;
-    if (tid < F && ps.first) {
+    if (ps.first) {
         const int T = s_toff[ps.r + 1] - s_toff[ps.r];
         int t, p;
         if (ps.cnt > 1) {
@@ -339,7 +348,7 @@ __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int 
         } else {
             in_free_slot(ps.pn, T, s_c[1][ps.r], t, p);
         }
-        *t_rel = t;
+        t_rel = t;
         const int64_t row0 = (tbase + s_toff[ps.r] + t) * 16 + p;
         tfeat[row0] = (ps.f - ps.r_lo) * row_bytes;
         tsrc[row0] = (ps.rank << 10) | (ps.cnt << 1);
@@ -361,6 +370,7 @@ __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int 
         tfeat[(tbase + t) * 16 + p] = (trash_row + (p & (kTrashRows - 1))) * row_bytes;
         tsrc[(tbase + t) * 16 + p] = 0;
     }
+    return t_rel;
 }
 
 // The tile table of one range for the pinned layout, made by one thread from the
@@ -369,34 +379,37 @@ __device__ __forceinline__ void plan_in_tile(const PlanSlot& ps, int64_t g, int 
 // tiles 8), pinned singles follow a tile's duplicated rows, and the other
 // singles are dealt over the tiles in turn, round k giving one row to every tile
 // with at least k free rows (appended tiles take 16 in order).  Writes the
-// range's tile count to *nt (over kPairRangeTiles: the pinned layout fails).
+// range's tile count to *nt (over TT, the tiles tracked: the pinned layout fails).
+template <int TT>
 struct PairTables {
-    int cb[kPairRanges][kPairRangeTiles];    // first unpinned-dup ordinal of the tile
-    int ce[kPairRanges][kPairRangeTiles];    // one past its last
-    int base[kPairRanges][kPairRangeTiles];  // rows of the tile's duplicated features
-    int fr[kPairRanges][kPairRangeTiles];    // rows free for the dealt singles
+    int cb[kPairRanges][TT];    // first unpinned-dup ordinal of the tile
+    int ce[kPairRanges][TT];    // one past its last
+    int base[kPairRanges][TT];  // rows of the tile's duplicated features
+    int fr[kPairRanges][TT];    // rows free for the dealt singles
     int S[kPairRanges][17];                  // dealt singles in rounds 1..k
     int nt1[kPairRanges];                    // tiles before the dealt singles' appended ones
 };
 
+template <int TT>
 __device__ __forceinline__ void pair_range_table(int r, int c0, int nd, int maxpin,
-                                                 const int* __restrict__ pd, const int* __restrict__ rs,
-                                                 PairTables& tb, int* nt) {
+                                                 const int* __restrict__ pins,
+                                                 PairTables<TT>& tb, int* nt) {
     int npd = 0, nrs = 0, need_ok = 1;
-    int p2[kPairRangeTiles], q1[kPairRangeTiles];
+    int p2[TT], q1[TT];
 #pragma unroll
-    for (int t = 0; t < kPairRangeTiles; ++t) {
-        p2[t] = 2 * pd[t];
-        q1[t] = rs[t];
-        npd += pd[t];
-        nrs += rs[t];
+    for (int t = 0; t < TT; ++t) {
+        const int pd = pins[t] & 0xFFFF;
+        p2[t] = 2 * pd;
+        q1[t] = pins[t] >> 16;
+        npd += pd;
+        nrs += q1[t];
         need_ok &= p2[t] + q1[t] <= 16;
     }
     const int nt0 = max((c0 + nd + 15) / 16, maxpin + 1);
     const int M = nd - npd, U = (c0 - nd) - nrs;
     int C = 0, nt1 = nt0;
 #pragma unroll
-    for (int t = 0; t < kPairRangeTiles; ++t) {
+    for (int t = 0; t < TT; ++t) {
         const int cap = t < nt0 ? (16 - p2[t] - q1[t]) / 2 : 8;
         const int u = min(max(M - C, 0), cap);
         if (t >= nt0 && u > 0) nt1 = t + 1;
@@ -407,138 +420,165 @@ __device__ __forceinline__ void pair_range_table(int r, int c0, int nd, int maxp
         tb.base[r][t] = p2[t];
         q1[t] = t < nt1 ? 16 - p2[t] - q1[t] : 0;        // free rows (after nt1 is final below)
     }
-    bool ok = need_ok && nt0 <= kPairRangeTiles && M <= C;
+    bool ok = need_ok && nt0 <= TT && M <= C;
     int S = 0;
     tb.S[r][0] = 0;
 #pragma unroll
     for (int k = 1; k <= 16; ++k) {
 #pragma unroll
-        for (int t = 0; t < kPairRangeTiles; ++t) S += (t < nt1 && q1[t] >= k) ? 1 : 0;
+        for (int t = 0; t < TT; ++t) S += (t < nt1 && q1[t] >= k) ? 1 : 0;
         tb.S[r][k] = S;
     }
 #pragma unroll
-    for (int t = 0; t < kPairRangeTiles; ++t) tb.fr[r][t] = t < nt1 ? q1[t] : 0;
+    for (int t = 0; t < TT; ++t) tb.fr[r][t] = t < nt1 ? q1[t] : 0;
     tb.nt1[r] = nt1;
     const int nt2 = nt1 + (U > S ? (U - S + 15) / 16 : 0);
-    *nt = ok ? nt2 : kPairRangeTiles + 1;
+    *nt = ok ? nt2 : TT + 1;
 }
 
-// NT threads, at least one per slot.
-template <int NT>
-__global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(const int32_t* __restrict__ idx,
-                                                               int* __restrict__ tfeat,
-                                                               int* __restrict__ tsrc,
-                                                               int* __restrict__ perm,
-                                                               int* __restrict__ meta, int F, int D,
-                                                               int ndr, int Dc, int Tcap,
-                                                               int row_bytes, int trash_row,
-                                                               int64_t Gc) {
-    __shared__ __align__(16) int s_idx[kPlanWindow][NT];
-    __shared__ __align__(16) int s_flag[kPlanWindow][NT];
-    __shared__ __align__(16) int s_ftile[kPlanWindow][NT];   // tile of the slot's feature (first occurrences)
-    __shared__ int s_c[2][kMaxRanges];
+// NT threads, at least one per slot.  What bounds it is the chain of a window's
+// groups, each laid out by where the one before put its features, and the
+// latency of every step in it.  So all that does not depend on the layouts comes
+// before the chain, for the window's groups side by side: the rows' analysis, and
+// each feature's slot in the window's earlier groups.  The chain keeps a lookup of
+// the pinned tiles, the rank scan, the tile table and the placement.
+// Measured (us; the groups in turn with a tile table of 24 in every plan -> this;
+// G = 64, D = 768 - 1500): 46 -> 37 at O = 20,011, F = 64, the latency of one window; 97
+// -> 60 at O = 670,091, F = 64; 256 -> 180 at O = 400,001, F = 144, four ranges; 77 -> 73 at
+// O = 131,073, F = 128 (24 tiles).  NT threads for each of the window's groups took 27
+// us at O = 20,011 but 485 at O = 400,001, F = 144, as most of its waves wait.
+template <int NT, int TT>
+__global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(
+    const int32_t* __restrict__ idx, int* __restrict__ tfeat, int* __restrict__ tsrc,
+    int* __restrict__ perm, int* __restrict__ meta, int F, int D, int ndr, int Dc, int Tcap,
+    int row_bytes, int trash_row, int64_t Gc) {
+    constexpr int W = kPlanWindow;
+    static_assert(W == 3 && NT >= 64 && kPairRanges <= 64, "src below; the table's threads");
+    __shared__ __align__(16) int s_idx[W][NT];
+    __shared__ __align__(16) int s_flag[W][NT];
+    __shared__ short s_ftile[(W - 1) * NT];        // tile of the slot's feature (first occurrences)
+    __shared__ __align__(16) short s_pin[NT];      // the slot's pinned tile, or -1
+    __shared__ int s_c[W][2][kMaxRanges];
+    // of the window's later groups, per range: pinned features per tile (duplicated
+    // ones in bits 0 - 15, single ones from bit 16), rows used per tile, last tile
+    __shared__ int s_pins[W - 1][kPairRanges][TT];
+    __shared__ int s_used[W - 1][kPairRanges][TT];
+    __shared__ int s_maxpin[W - 1][kPairRanges];
+    __shared__ int s_fail[W];
+    __shared__ PairTables<TT> s_tb;
+    __shared__ int s_nt[kPairRanges];              // tiles per range
     __shared__ int s_toff[kMaxRanges + 1];
-    __shared__ int s_pd[kPairRanges][kPairRangeTiles];        // pinned duplicated features per tile
-    __shared__ int s_rs[kPairRanges][kPairRangeTiles];        // pinned single features per tile
-    __shared__ int s_used[kPairRanges][kPairRangeTiles];      // rows used per tile
-    __shared__ int s_maxpin[kPairRanges];
-    __shared__ __align__(16) short s_pin[NT];                // the slot's pinned tile, or -1
-    __shared__ PairTables s_tb;
-    __shared__ int s_nt[kPairRanges];                         // tiles per range
-    __shared__ int s_fail;
     const int tid = threadIdx.x;
-    for (int j = 0; j < kPlanWindow; ++j) {
-        const int64_t g = kPlanWindow * (int64_t)blockIdx.x + j;
-        if (g >= Gc) return;  // (uniform)
-        for (int i = tid; i < 2 * kMaxRanges; i += NT) (&s_c[0][0])[i] = 0;
-        for (int i = tid; i < kPairRanges * kPairRangeTiles; i += NT) {
-            (&s_pd[0][0])[i] = 0;
-            (&s_rs[0][0])[i] = 0;
-            (&s_used[0][0])[i] = 0;
+    const int64_t g0 = W * (int64_t)blockIdx.x;
+    const int F4 = (F + 3) & ~3;
+    for (int i = tid; i < W * 2 * kMaxRanges; i += NT) (&s_c[0][0][0])[i] = 0;
+    for (int i = tid; i < (W - 1) * kPairRanges * TT; i += NT) {
+        (&s_pins[0][0][0])[i] = 0;
+        (&s_used[0][0][0])[i] = 0;
+    }
+    if (tid < (W - 1) * kPairRanges) (&s_maxpin[0][0])[tid] = -1;
+    if (tid < W) s_fail[tid] = tid == 0 || ndr > kPairRanges;
+    PlanSlot slots[W];
+    plan_analyse<W, NT>(idx, g0, Gc, F, D, Dc, s_idx, s_flag, s_c, perm, slots);
+    // of the later groups, the first slot of the thread's feature in the latest of the
+    // window's earlier groups that holds it: the slot whose tile it is pinned to
+    int src0 = -1, src1 = -1, src2 = -1;
+    {
+        int m10 = NT, m20 = NT, m21 = NT;
+        auto find = [&](int& m, const int4& v, int f, int k) {
+            m = min(m, v.x == f ? k : v.y == f ? k + 1 : v.z == f ? k + 2 : v.w == f ? k + 3 : NT);
+        };
+#pragma unroll 2
+        for (int k4 = 0; k4 < F4 / 4; ++k4) {
+            const int4 v0 = reinterpret_cast<const int4*>(s_idx[0])[k4];
+            const int4 v1 = reinterpret_cast<const int4*>(s_idx[1])[k4];
+            find(m10, v0, slots[1].f, 4 * k4);
+            find(m20, v0, slots[2].f, 4 * k4);
+            find(m21, v1, slots[2].f, 4 * k4);
         }
-        if (tid < kPairRanges) s_maxpin[tid] = -1;
-        if (tid == 0) s_fail = j == 0 || ndr > kPairRanges;
-        __syncthreads();
-        PlanSlot ps = plan_analyse(idx, g, F, D, Dc, s_idx[j], s_flag[j], s_c, perm);
-        const bool mine = tid < F && ps.first;
+        if (slots[1].first && m10 < NT) src1 = m10;
+        if (slots[2].first) src2 = m21 < NT ? NT + m21 : m20 < NT ? m20 : -1;
+    }
+    for (int j = 0; j < W; ++j) {
+        const int64_t g = g0 + j;
+        if (g >= Gc) return;  // (uniform)
+        PlanSlot ps = slots[0];
+        const int src = src0;
+        slots[0] = slots[1];  // the next group's in turn, without indexed registers
+        slots[1] = slots[2];
+        src0 = src1;
+        src1 = src2;
+        const bool mine = ps.first;
         const bool dup = ps.cnt > 1;
-        // each feature the window's earlier groups hold pinned to the tile of
-        // the latest of them that holds it
-        int pin = -1;
-        if (mine) {
-            const int F4 = (F + 3) & ~3;
-            for (int jj = j - 1; jj >= 0 && pin < 0; --jj) {
-                const int4* v4 = reinterpret_cast<const int4*>(s_idx[jj]);
-                const int4* t4 = reinterpret_cast<const int4*>(s_ftile[jj]);
+        int pin = -1, rank = 0;
+        if (j > 0) {
+            if (src >= 0) pin = s_ftile[src];
+            s_pin[tid] = (short)pin;
+            if (pin >= TT) {
+                atomicOr(&s_fail[j], 1);
+            } else if (pin >= 0 && !s_fail[j]) {
+                atomicAdd(&s_pins[j - 1][ps.r][pin], dup ? 1 : 1 << 16);
+                atomicMax(&s_maxpin[j - 1][ps.r], pin);
+            }
+            __syncthreads();
+            // the tile table, by the last wave's threads
+            const int tr = tid - (NT - 64);
+            if (tr >= 0 && tr < ndr && !s_fail[j]) {
+                int nt;
+                pair_range_table<TT>(tr, s_c[j][0][tr], s_c[j][1][tr], s_maxpin[j - 1][tr],
+                                     s_pins[j - 1][tr], s_tb, &nt);
+                s_nt[tr] = nt;
+                if (nt > TT) atomicOr(&s_fail[j], 1);
+            }
+            // the slot's rank in its class: pinned rows by slot among their tile's,
+            // unpinned duplicated features by slot, unpinned singles by residue key
+            if (mine && !s_fail[j]) {
+                const int key = (((ps.f - ps.r_lo) & 15) << 16) | (ps.f - ps.r_lo);
+                const bool by_key = pin < 0 && !dup;
+                auto count = [&](int k, int v, int fl, int pk) {
+                    const int kk = (((v - ps.r_lo) & 15) << 16) | (v - ps.r_lo);
+                    const bool same = (fl & 1) && v >= ps.r_lo && v < ps.r_lo + Dc &&
+                                      ((fl & 2) != 0) == dup && pk == pin;
+                    rank += same && (by_key ? kk < key : k < tid);
+                };
+                const int4* v4 = reinterpret_cast<const int4*>(s_idx[j]);
+                const int4* f4 = reinterpret_cast<const int4*>(s_flag[j]);
+                const short4* p4 = reinterpret_cast<const short4*>(s_pin);
 #pragma unroll 4
                 for (int k4 = 0; k4 < F4 / 4; ++k4) {
-                    const int4 v = v4[k4], t = t4[k4];
-                    pin = max(pin, v.x == ps.f ? t.x : -1);  // one slot of a group holds the tile
-                    pin = max(pin, v.y == ps.f ? t.y : -1);
-                    pin = max(pin, v.z == ps.f ? t.z : -1);
-                    pin = max(pin, v.w == ps.f ? t.w : -1);
+                    const int4 v = v4[k4], fl = f4[k4];
+                    const short4 pk = p4[k4];
+                    count(4 * k4, v.x, fl.x, pk.x);
+                    count(4 * k4 + 1, v.y, fl.y, pk.y);
+                    count(4 * k4 + 2, v.z, fl.z, pk.z);
+                    count(4 * k4 + 3, v.w, fl.w, pk.w);
                 }
             }
+            __syncthreads();
         }
-        s_pin[tid] = (short)pin;
-        if (mine && pin >= 0 && !s_fail) {
-            if (pin >= kPairRangeTiles) {
-                atomicOr(&s_fail, 1);
-            } else {
-                atomicAdd(dup ? &s_pd[ps.r][pin] : &s_rs[ps.r][pin], 1);
-                atomicMax(&s_maxpin[ps.r], pin);
-            }
-        }
-        __syncthreads();
-        // the slot's rank in its class: pinned rows by slot among their tile's,
-        // unpinned duplicated features by slot, unpinned singles by residue key
-        int rank = 0;
-        if (mine && !s_fail) {
-            const int key = (((ps.f - ps.r_lo) & 15) << 16) | (ps.f - ps.r_lo);
-            const bool by_key = pin < 0 && !dup;
-            auto count = [&](int k, int v, int fl, int pk) {
-                const int kk = (((v - ps.r_lo) & 15) << 16) | (v - ps.r_lo);
-                const bool same = (fl & 1) && v >= ps.r_lo && v < ps.r_lo + Dc &&
-                                  ((fl & 2) != 0) == dup && pk == pin;
-                rank += same && (by_key ? kk < key : k < tid);
-            };
-            const int4* v4 = reinterpret_cast<const int4*>(s_idx[j]);
-            const int4* f4 = reinterpret_cast<const int4*>(s_flag[j]);
-            const short4* p4 = reinterpret_cast<const short4*>(s_pin);
-            const int F4 = (F + 3) & ~3;
-#pragma unroll 4
-            for (int k4 = 0; k4 < F4 / 4; ++k4) {
-                const int4 v = v4[k4], fl = f4[k4];
-                const short4 pk = p4[k4];
-                count(4 * k4, v.x, fl.x, pk.x);
-                count(4 * k4 + 1, v.y, fl.y, pk.y);
-                count(4 * k4 + 2, v.z, fl.z, pk.z);
-                count(4 * k4 + 3, v.w, fl.w, pk.w);
-            }
-        }
-        if (tid < ndr && !s_fail) {
-            int nt;
-            pair_range_table(tid, s_c[0][tid], s_c[1][tid], s_maxpin[tid], s_pd[tid], s_rs[tid], s_tb, &nt);
-            s_nt[tid] = nt;
-            if (nt > kPairRangeTiles) atomicOr(&s_fail, 1);
-        }
-        __syncthreads();
-        if (tid == 0 && !s_fail) {
-            int t = 0;
-            for (int rr = 0; rr < ndr; ++rr) {
+        // the ranges' first tiles: of the pinned layout or, where there is none, of
+        // the group's own
+        auto offsets = [&](bool alone) {
+            for (int rr = tid; rr <= ndr; rr += NT) {
+                int t = 0;
+                for (int q = 0; q < rr; ++q) t += alone ? range_tiles(s_c[j], q) : s_nt[q];
                 s_toff[rr] = t;
-                t += s_nt[rr];
             }
-            s_toff[ndr] = t;
-            if (t > Tcap) s_fail = 1;
+            __syncthreads();
+        };
+        bool fail = s_fail[j] != 0;
+        offsets(fail);
+        if (!fail && s_toff[ndr] > Tcap) {  // (uniform)
+            fail = true;
+            __syncthreads();
+            offsets(true);
         }
-        __syncthreads();
-        if (s_fail) {  // (uniform) laid out on its own; past the window's first, the barrier kept
-            int tr = -1;
+        if (fail) {  // laid out on its own; past the window's first, the barrier kept
             plan_keys(ps, F, Dc, s_idx[j], s_flag[j]);
-            plan_in_tile<NT>(ps, g, F, ndr, Tcap, row_bytes, trash_row, j == 0 ? 0u : kMetaUnpaired, s_c,
-                         s_toff, tfeat, tsrc, meta, &tr);
-            s_ftile[j][tid] = mine ? tr : -1;
+            const int t =
+                plan_in_tile<NT>(ps, g, ndr, Tcap, row_bytes, trash_row,
+                                 j == 0 ? 0u : kMetaUnpaired, s_c[j], s_toff, tfeat, tsrc, meta);
+            if (j < W - 1) s_ftile[j * NT + tid] = (short)t;
             __syncthreads();
             continue;
         }
@@ -548,17 +588,17 @@ __global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(const int32_t* __r
             m[1] = s_toff[rr + 1];
         }
         const int64_t tbase = g * Tcap;
-        s_ftile[j][tid] = -1;
+        int t = -1;
         if (mine) {
             const int r = ps.r;
-            int t, p;
+            int p;
             if (pin >= 0) {
                 t = pin;
                 p = dup ? 2 * rank : s_tb.base[r][t] + rank;
             } else if (dup) {
                 t = 0;
                 while (rank >= s_tb.ce[r][t]) ++t;  // rank < the range's unpinned dups <= ce[nt-1]
-                p = s_pd[r][t] * 2 + 2 * (rank - s_tb.cb[r][t]);
+                p = (s_pins[j - 1][r][t] & 0xFFFF) * 2 + 2 * (rank - s_tb.cb[r][t]);
             } else if (rank < s_tb.S[r][16]) {
                 int k = 1;
                 while (rank >= s_tb.S[r][k]) ++k;
@@ -576,8 +616,7 @@ __global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(const int32_t* __r
                 t = s_tb.nt1[r] + q / 16;
                 p = q % 16;
             }
-            atomicAdd(&s_used[r][t], dup ? 2 : 1);
-            s_ftile[j][tid] = t;
+            atomicAdd(&s_used[j - 1][r][t], dup ? 2 : 1);
             const int64_t row0 = (tbase + s_toff[r] + t) * 16 + p;
             tfeat[row0] = (ps.f - ps.r_lo) * row_bytes;
             tsrc[row0] = (ps.rank << 10) | (ps.cnt << 1);
@@ -586,41 +625,45 @@ __global__ __launch_bounds__(NT) void bwdf_plan_window_kernel(const int32_t* __r
                 tsrc[row0 + 1] = (ps.rank << 10) | (ps.cnt << 1) | 1;
             }
         }
+        if (j < W - 1) s_ftile[j * NT + tid] = (short)t;
         __syncthreads();
+        // padding rows (s_toff changes after two more barriers)
         const int nslots = s_toff[ndr] * 16;
         for (int i = tid; i < nslots; i += NT) {
-            const int t = i / 16, p = i % 16;
+            const int tt = i / 16, p = i % 16;
             int rr = 0;
-            while (t >= s_toff[rr + 1]) ++rr;
-            if (p < s_used[rr][t - s_toff[rr]]) continue;
-            tfeat[(tbase + t) * 16 + p] = (trash_row + (p & (kTrashRows - 1))) * row_bytes;
-            tsrc[(tbase + t) * 16 + p] = 0;
+            while (tt >= s_toff[rr + 1]) ++rr;
+            if (p < s_used[j - 1][rr][tt - s_toff[rr]]) continue;
+            tfeat[(tbase + tt) * 16 + p] = (trash_row + (p & (kTrashRows - 1))) * row_bytes;
+            tsrc[(tbase + tt) * 16 + p] = 0;
         }
-        __syncthreads();
     }
 }
 
 // The plan of p: the staged build's in windows of groups, the others per group.
 void launch_plan(const int32_t* idx, int* tfeat, int* tsrc, int* perm, int* meta, int64_t F,
                  int64_t D, const BwdFPlan& p, hipStream_t st) {
-    // one thread per slot: the plan's time goes to its barriers and serial parts,
-    // which idle waves only lengthen (256 threads at O = 670,091, F = 64: about
-    // 240 us, 64 threads 104)
+    // one thread per slot: idle waves would only lengthen the barriers
     const dim3 windows((unsigned)ceil_div(p.Gc, (int64_t)kPlanWindow));
-#define HASTE_PLAN_WIN(NT)                                                                      \
-    bwdf_plan_window_kernel<NT><<<windows, dim3(NT), 0, st>>>(                                   \
+    const bool half = p.tiles < kStagedTiles;
+#define HASTE_PLAN_WIN(NT, HALF)                                                                \
+    bwdf_plan_window_kernel<NT, pair_range_tiles(HALF)><<<windows, dim3(NT), 0, st>>>(          \
         idx, tfeat, tsrc, perm, meta, (int)F, (int)D, (int)p.ndr, (int)p.Dc, (int)p.Tcap,       \
         acc_stride((int)p.BT) * 4, (int)p.DCMAX, p.Gc)
-    if (p.staged && F <= 64)
-        HASTE_PLAN_WIN(64);
-    else if (p.staged && F <= 128)
-        HASTE_PLAN_WIN(128);
-    else if (p.staged)
-        HASTE_PLAN_WIN(256);
-    else
+    if (p.staged && F <= 64) {
+        if (half) HASTE_PLAN_WIN(64, true);
+        else HASTE_PLAN_WIN(64, false);
+    } else if (p.staged && F <= 128) {
+        if (half) HASTE_PLAN_WIN(128, true);
+        else HASTE_PLAN_WIN(128, false);
+    } else if (p.staged) {
+        if (half) HASTE_PLAN_WIN(256, true);
+        else HASTE_PLAN_WIN(256, false);
+    } else {
         bwdf_plan_kernel<<<dim3((unsigned)p.Gc), dim3(256), 0, st>>>(
             idx, tfeat, tsrc, perm, meta, (int)F, (int)D, (int)p.ndr, (int)p.Dc, (int)p.Tcap,
             acc_stride((int)p.BT) * 4, (int)p.DCMAX);
+    }
 #undef HASTE_PLAN_WIN
 }
 

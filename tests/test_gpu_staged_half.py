@@ -29,11 +29,17 @@ def test_two_waves_to_a_tile(dev, B, D, O, G, F, mode):
     torch.testing.assert_close(dXT.cpu(), ref, **TOL32)
 
 
-@pytest.mark.parametrize("mode", ["random", "dups"])
+# front: in some windows of groups a range holds every feature, more tiles than the
+# plan's window layout tracks
+@pytest.mark.parametrize("mode", ["random", "dups", "front"])
 @pytest.mark.parametrize("B,D,O,G,F", HALF_CASES)
 def test_every_build_with_two_waves_to_a_tile(dev, B, D, O, G, F, mode):
     """One shape per build (tests/test_abi.py checks the coverage), whatever the default is."""
-    x, W, bias, idx, dY = make_case(B, D, O, G, F, idx_mode=mode, seed=D)
+    x, W, bias, idx, dY = make_case(B, D, O, G, F, seed=D,
+                                    idx_mode="random" if mode == "front" else mode)
+    if mode == "front":
+        idx[1::4] = torch.randperm(F).to(torch.int32)
+        idx[2::4] = torch.randperm(F).to(torch.int32)
     prev = _lib.lib().haste_ffi_bwd_features_set_build(3)
     try:
         dXT = _C.ffi_backward_features_cuda(x.t().contiguous().to(dev), W.to(dev), idx.to(dev),
