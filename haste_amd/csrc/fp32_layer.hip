@@ -11,19 +11,23 @@ namespace {
 constexpr int kThreads = 256;
 
 // out[r, 8p .. 8p+7] = RNE(in[r, ...]) (0 past the row): a thread one 8-element
-// piece.  in's rows start on 4-byte boundaries only (its loads are unaligned
-// 16-byte ones), out's on 128-byte lines, so that the backward kernels take
-// their aligned builds: torch's cast left rows at in's stride, and backward to
-// features took 51 us and the weight gradient 36.5 where they now take
-// F32_FIGS (B = 256, O = 131,073, G = 32, F = 64), at the cost of the cast alone.
+// piece, 2^tx threads to a row, so that short rows share a workgroup (60,000 rows
+// of 100: 28 us with a workgroup to a row, below the launch's 9 here).  in's rows start on
+// 4-byte boundaries only (its loads are unaligned 16-byte ones), out's on
+// 128-byte lines, so that the backward kernels take their aligned builds: torch's
+// cast left rows at in's stride, where the weight gradient took 36.5 us, now 29.8
+// (B = 256, O = 131,073, G = 32, F = 64), at the cost of torch's cast (28 us, 7.2 TB/s).
 __global__ __launch_bounds__(kThreads) void cast_rows_f16_kernel(const float* __restrict__ in,
                                                                  int64_t ldi,
                                                                  uint16_t* __restrict__ out,
-                                                                 int64_t ldo, int64_t cols) {
+                                                                 int64_t ldo, int64_t rows,
+                                                                 int64_t cols, int tx) {
     typedef f32x4 __attribute__((aligned(4))) f32x4_u;
-    const int64_t c = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 8;
-    if (c >= cols) return;
-    const float* p = in + (int64_t)blockIdx.y * ldi + c;
+    const int x = threadIdx.x & ((1 << tx) - 1), y = threadIdx.x >> tx;
+    const int64_t r = (int64_t)blockIdx.y * (kThreads >> tx) + y;
+    const int64_t c = (((int64_t)blockIdx.x << tx) + x) * 8;
+    if (r >= rows || c >= cols) return;
+    const float* p = in + r * ldi + c;
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
     if (c + 8 <= cols) {
         a = *reinterpret_cast<const f32x4_u*>(p);
@@ -35,7 +39,7 @@ __global__ __launch_bounds__(kThreads) void cast_rows_f16_kernel(const float* __
             b[e] = c + 4 + e < cols ? p[4 + e] : 0.f;
         }
     }
-    *reinterpret_cast<u32x4*>(out + (int64_t)blockIdx.y * ldo + c) =
+    *reinterpret_cast<u32x4*>(out + r * ldo + c) =
         u32x4{pack2_rne<F16>(a[0], a[1]), pack2_rne<F16>(a[2], a[3]), pack2_rne<F16>(b[0], b[1]),
               pack2_rne<F16>(b[2], b[3])};
 }
@@ -114,10 +118,14 @@ extern "C" int haste_cast_rows_f16(const float* in, int64_t ldi, uint16_t* out, 
                         haste::aligned16(out) && reinterpret_cast<uintptr_t>(in) % 4 == 0,
                     "%s: null pointer, short stride or misaligned rows (ldi=%lld ldo=%lld "
                     "cols=%lld)", fn, (long long)ldi, (long long)ldo, (long long)cols);
-    const int64_t bx = haste::ceil_div(cols, (int64_t)8 * haste::kThreads);
+    int tx = 0;
+    while (tx < 8 && (int64_t)8 << tx < cols) ++tx;
+    const int64_t bx = haste::ceil_div(cols, (int64_t)8 << tx);
+    const int64_t by = haste::ceil_div(rows, (int64_t)haste::kThreads >> tx);
     HASTE_CHECK_ARG(rows < 65536 && bx < 0x7FFFFFFF, "%s: matrix too large", fn);
-    haste::cast_rows_f16_kernel<<<dim3((unsigned)bx, (unsigned)rows), dim3(haste::kThreads), 0,
-                                  static_cast<hipStream_t>(stream)>>>(in, ldi, out, ldo, cols);
+    haste::cast_rows_f16_kernel<<<dim3((unsigned)bx, (unsigned)by), dim3(haste::kThreads), 0,
+                                  static_cast<hipStream_t>(stream)>>>(in, ldi, out, ldo, rows, cols,
+                                                                      tx);
     HASTE_CHECK_LAUNCH(fn);
     return HASTE_OK;
 }

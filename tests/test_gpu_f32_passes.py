@@ -40,7 +40,11 @@ def test_sgd_f32(dev, wd, mu):
 
 
 @pytest.mark.parametrize("B,O,ld,off", [(1, 2, 2, 0), (3, 7, 7, 0), (5, 8, 8, 0), (4, 2049, 2049, 0),
-                                        (7, 131, 140, 3), (64, 4096, 4096, 0)])
+                                        (7, 131, 140, 3), (64, 4096, 4096, 0),
+                                        # rows sharing a workgroup: its last one partly filled,
+                                        # widths around a power of two of pieces
+                                        (600, 20, 20, 0), (257, 9, 9, 0), (33, 64, 67, 1),
+                                        (5, 1025, 1025, 0), (3, 2047, 2047, 2)])
 def test_compute_rows(dev, B, O, ld, off):
     buf = torch.randn(B * ld + 16, device=dev) * 100
     buf[off:off + 2] = torch.tensor([1e6, float("nan")], device=dev)
