@@ -87,7 +87,7 @@ def compute_rows(t: torch.Tensor) -> Tuple[torch.Tensor, int]:
     """grad_rows of grad_output as the kernels compute with it: fp32 rows are
     rounded to fp16 into a buffer whose rows start on 128-byte lines."""
     if t.dtype != torch.float32 or t.shape[0] >= 65536 or t.shape[1] < 2 or t.stride(1) != 1 \
-            or t.stride(0) < t.shape[1] or t.numel() == 0 or not t.is_cuda \
+            or t.stride(0) < t.shape[1] or t.numel() == 0 or not t.is_cuda or t.is_neg() \
             or (t.shape[1] % 64 == 0 and t.is_contiguous()):  # torch's cast has such rows
         return grad_rows(f16_compute(t))
     ld = round64(t.shape[1])

@@ -52,3 +52,9 @@ def test_compute_rows(dev, B, O, ld, off):
     rows, ldo = _C.compute_rows(t)
     assert ldo % 64 == 0 and rows.data_ptr() % 16 == 0 and rows.stride() == (ldo, 1)
     assert torch.equal(rows.nan_to_num(7.0), t.to(torch.float16).nan_to_num(7.0))
+
+
+def test_compute_rows_of_a_negated_view(dev):
+    t = torch._neg_view(torch.randn(5, 37, device=dev))
+    rows, _ = _C.compute_rows(t)
+    assert torch.equal(rows, (-torch._neg_view(t)).to(torch.float16))
