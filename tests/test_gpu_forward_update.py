@@ -79,3 +79,15 @@ def test_rows_off_16_bytes_and_dY_in_the_logits(dev):
     b.backward_features(b.logits_buf, b.ldo, defer_dx=True)
     b.backward_weights_sgd(b.logits_buf, b.ldo)
     assert torch.equal(a.logits, b.logits) and torch.equal(a.W, b.W) and torch.equal(a.dX, b.dX)
+
+
+def test_step_is_its_parts_with_streamed_dY(dev):
+    """dY just above the size from which the launch loads it without keeping it in the caches."""
+    B, D, O, G, F = 512, 300, 270001, 64, 64
+    x, W, bias, idx, dY = case(dev, B, D, O, G, F)
+    ld = (O + 7) // 8 * 8
+    dY = dY[:, :ld].contiguous()
+    assert (256 << 20) < dY.numel() * 2 < (272 << 20)
+    a, b = both(dev, x, W, bias, idx, G, [(dY, ld)] * 2)
+    assert torch.equal(a.logits, b.logits) and torch.equal(a.dX, b.dX)
+    assert torch.equal(a.W, b.W) and torch.equal(a.bias, b.bias)
