@@ -177,7 +177,8 @@ class FFITrainStep:
         """A training step with the loss fused into the forward: forward + BCE
         gradient -> backward to features (dX) -> fused weight/bias gradient +
         SR-SGD.  Returns the loss (0-d fp32 device tensor) of the step's forward."""
-        if self.grad_dtype != torch.float32 or labels.numel() > 1 << 21:
+        if (self.grad_dtype != torch.float32 or labels.numel() > 1 << 21
+                or self._replaced("forward_bce", "backward_weights_sgd")):
             loss = self.forward_bce(x, labels)
             self.backward_features(self.dY_buf, self.ldo, defer_dx=True)
             self.backward_weights_sgd(self.dY_buf, self.ldo)
@@ -212,6 +213,12 @@ class FFITrainStep:
         self._dx_pending = False
         self._weights_updated(True)
         return self.loss_buf
+
+    def _replaced(self, *names: str) -> bool:
+        """Whether a subclass, a patch or an attribute replaces one of these methods: a
+        step then calls them instead of the launches that join them."""
+        cls, own = type(self), self.__dict__
+        return any(n in own or getattr(cls, n) is not _JOINED[n] for n in names)
 
     def _check_dY(self, dY: torch.Tensor, lddy: int) -> None:
         _C.require_device(dY, "dY")
@@ -339,8 +346,9 @@ class FFITrainStep:
         bit-identical to forward, backward_features, backward_weights_sgd in turn).
         A dY that shares memory with the logits is read after they are written."""
         lo, hi = self.logits_buf.data_ptr(), dY.data_ptr()
-        if (self.grad_dtype != torch.float32 or (hi < lo + self.logits_buf.numel() * 2
-                                                 and lo < hi + dY.numel() * dY.element_size())):
+        if (self.grad_dtype != torch.float32 or self._replaced("forward", "backward_weights_sgd")
+                or (hi < lo + self.logits_buf.numel() * 2
+                    and lo < hi + dY.numel() * dY.element_size())):
             self.forward(x)
             self.backward_features(dY, lddy, defer_dx=True)
             self.backward_weights_sgd(dY, lddy)
@@ -357,3 +365,7 @@ class FFITrainStep:
                   _C.stream_of(self.W))
         self._dx_pending = False
         self._weights_updated(True)
+
+
+# the methods whose work step and step_bce do in joined launches
+_JOINED = {n: vars(FFITrainStep)[n] for n in ("forward", "forward_bce", "backward_weights_sgd")}
