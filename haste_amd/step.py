@@ -218,7 +218,10 @@ class FFITrainStep:
         """Whether a subclass, a patch or an attribute replaces one of these methods: a
         step then calls them instead of the launches that join them."""
         cls, own = type(self), self.__dict__
-        return any(n in own or getattr(cls, n) is not _JOINED[n] for n in names)
+        for n in names:
+            if n in own or getattr(cls, n) is not _JOINED[n]:
+                return True
+        return False
 
     def _check_dY(self, dY: torch.Tensor, lddy: int) -> None:
         _C.require_device(dY, "dY")
