@@ -84,6 +84,7 @@ SIGNATURES = {
                                                              _P, _F32, _F32, _F32, _I32, _I32,
                                                              _P, _P, _U64, _P, _I64, _I64, _I64,
                                                              _I64, _I64, _I64, _I32, _P]),
+    "haste_ffi_forward_bwd_weights_joined": (ctypes.c_int, [_P, _I64, _I64, _I64, _I64, _I64, _I64]),
     "haste_ffi_forward_bwd_weights_sgd_dx": (ctypes.c_int, [_P, _P, _I64, _P, _I64, _P, _P, _P, _P,
                                                             _P, _I64, _F32, _F32, _F32, _I32,
                                                             _I32, _U64, _P, _P, _U64, _P, _I64,

@@ -716,6 +716,7 @@ int dispatch_g(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16
 // The SGD launch that also computes the logits (FWD kernels; defined in
 // ffi_forward_bwdw.hip), for the dY, logits stride and tile sizes it has builds for.
 bool fwd_sgd_fits(const void* dY, int64_t lddy, int64_t ldl, int64_t F, int64_t G);
+bool fwd_sgd_pays(int64_t lddy, int64_t B, int64_t F, int64_t O, int64_t G);
 int fwd_sgd_dispatch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16_t* dY,
                      int64_t lddy, int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
                      const SgdArgs& sg, hipStream_t st);

@@ -184,7 +184,7 @@ int bwdw_sgd(const char* fn, const int32_t* idx, const void* xT, int64_t ldx, co
             sg.rj = reduce_job(p, reinterpret_cast<const float*>(base + p.prep_bytes), dX, B, D,
                                dx_seed);
     }
-    if (logits != nullptr && fwd_sgd_fits(dY, lddy, ldl, F, G))
+    if (logits != nullptr && fwd_sgd_fits(dY, lddy, ldl, F, G) && fwd_sgd_pays(lddy, B, F, O, G))
         return fwd_sgd_dispatch(idx, static_cast<const uint16_t*>(xT), ldx,
                                 static_cast<const uint16_t*>(dY), lddy, B, D, F, O, G, sg,
                                 static_cast<hipStream_t>(stream));

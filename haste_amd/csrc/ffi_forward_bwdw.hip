@@ -38,6 +38,28 @@ bool fwd_sgd_fits(const void* dY, int64_t lddy, int64_t ldl, int64_t F, int64_t 
            64 * ldl * 2 <= kMaxRsrcBytes;
 }
 
+// Where the joined launch is faster than forward, backward to features and update
+// in turn.  Measured over some 2,500 shapes, B = 1 .. 1024 and O = 500 .. 1,600,000 (time of
+// the step, joined / in turn: mean, extremes; 1,450 of them also with other data
+// through the caches before each step, "cold"): 0.93 (0.72 - 1.07) where true, and
+// where not
+//  - under 100 groups with large batches and fan-ins, 1.02 (0.91 - 1.19): a group's
+//    chunks are one serial chain, longer in the joined kernel, on a chip that idles;
+//  - little work per group beside the joined kernel's fewer waves, with dY within the
+//    last-level cache: G = 128 with short rows from O = 300,000, 1.03 (0.97 - 1.08, cold
+//    1.02), and batches of one chunk at G = 64 with F half filling its tiles, 1.03 (0.99
+//    - 1.05, cold 1.05), or from 48M weights, 1.03 (0.97 - 1.07, cold 1.02).
+// A dY over that cache draws even (1.00, 0.86 - 1.09) where the same dY was read a step
+// ago, as its tail is then found there, and gains cold (0.95; 690 us in turn, 643 joined
+// at O = 670,091, G = F = 64, B = 512).
+bool fwd_sgd_pays(int64_t lddy, int64_t B, int64_t F, int64_t O, int64_t G) {
+    if (O < 100 * G) return B * F < 48 * 1024;
+    if (B * lddy * 2 > kMallBytes) return true;
+    if (G == 128) return F >= 64 || O < 300000;
+    const bool one_chunk = B <= 64 && F > 64 && F <= 128 && G > 16;
+    return !one_chunk || (O * F < 48000000 && (G == 32 || F > 112 || O < 50000));
+}
+
 int fwd_sgd_dispatch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const uint16_t* dY,
                      int64_t lddy, int64_t B, int64_t D, int64_t F, int64_t O, int64_t G,
                      const SgdArgs& sg, hipStream_t st) {
@@ -50,3 +72,8 @@ int fwd_sgd_dispatch(const int32_t* idx, const uint16_t* xT, int64_t ldx, const 
 }
 
 }  // namespace haste
+
+extern "C" int haste_ffi_forward_bwd_weights_joined(const void* dY, int64_t lddy, int64_t ldl,
+                                                    int64_t B, int64_t F, int64_t O, int64_t G) {
+    return haste::fwd_sgd_fits(dY, lddy, ldl, F, G) && haste::fwd_sgd_pays(lddy, B, F, O, G);
+}

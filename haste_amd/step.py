@@ -67,6 +67,7 @@ class FFITrainStep:
         self.code = _lib.DTYPE_BF16
         self.gcode = _C.dtype_code(grad_dtype)
         self._sgd_args = None
+        self._joins = {}     # step: whether rows of this stride and alignment take the joined launch
         # device_seed: the fused update's seed, read and advanced on the device
         self._seed_dev = (torch.tensor([self.seed], dtype=torch.int64, device=dev)
                           if device_seed else None)
@@ -344,12 +345,18 @@ class FFITrainStep:
     def step(self, x: torch.Tensor, dY: torch.Tensor, lddy: int) -> None:
         """Forward, backward to features (partials) and the fused weight/bias gradient +
         SR-SGD, whose launch also finishes dX.  dY is given, so the logits need
-        not come first: they are computed in the update's launch too, from the
-        weights and features it reads anyway (haste_ffi_forward_bwd_weights_sgd_dx;
-        bit-identical to forward, backward_features, backward_weights_sgd in turn).
+        not come first: at most sizes they are computed in the update's launch too,
+        from the weights and features it reads anyway
+        (haste_ffi_forward_bwd_weights_sgd_dx; bit-identical to forward,
+        backward_features, backward_weights_sgd in turn, which it is at the others).
         A dY that shares memory with the logits is read after they are written."""
         lo, hi = self.logits_buf.data_ptr(), dY.data_ptr()
-        if (self.grad_dtype != torch.float32 or self._replaced("forward", "backward_weights_sgd")
+        joins = self._joins.get((lddy, hi % 16))
+        if joins is None:
+            joins = self._joins[lddy, hi % 16] = _lib.lib().haste_ffi_forward_bwd_weights_joined(
+                hi, lddy, self.ldo, self.B, self.F, self.O, self.G)
+        if (not joins or self.grad_dtype != torch.float32
+                or self._replaced("forward", "backward_weights_sgd")
                 or (hi < lo + self.logits_buf.numel() * 2
                     and lo < hi + dY.numel() * dY.element_size())):
             self.forward(x)

@@ -348,14 +348,20 @@ int haste_sgd_sr_step_wt(uint16_t* W, const void* g, int32_t g_dtype, float* m, 
 /*
  * haste_ffi_forward with the weights and bias as they are on entry, and
  * haste_ffi_bwd_weights_sgd_dx (seed_dev not NULL: ..._dev_seed, seed unused), in
- * one launch where the sizes have a build for it (rows of dY on 16-byte
- * boundaries, G * F up to 128 * 128 or G < 128), else one after the other: for a
+ * one launch where the sizes have a build for it that is faster
+ * (haste_ffi_forward_bwd_weights_joined; rows of dY on 16-byte boundaries, G * F up to
+ * 128 * 128 or G < 128), else one after the other: for a
  * step whose dY does not depend on these logits, which reads each group's
  * weights and gathered features once instead of twice.  logits: [B, ldl] bf16,
  * ldl >= O and a multiple of 8, 16-byte aligned, must not overlap dY; the columns
  * from O up to the next multiple of 8 may be overwritten.  Bit-identical to the
  * two calls.  The bwd-features call comes first (before this call's update of W).
+ * ..._joined (host-only) is 1 where it is one launch; where not, haste_ffi_forward
+ * before the bwd-features call is the better order (the update then follows that
+ * call's read of dY).
  */
+int haste_ffi_forward_bwd_weights_joined(const void* dY, int64_t lddy, int64_t ldl, int64_t B,
+                                         int64_t F, int64_t O, int64_t G);
 int haste_ffi_forward_bwd_weights_sgd_dx(
     const int32_t* idx, const void* xT, int64_t ldx, const void* dY, int64_t lddy, uint16_t* W,
     uint16_t* bias, float* m_W, float* m_bias, uint16_t* logits, int64_t ldl, float lr, float wd,

@@ -267,6 +267,22 @@ def test_two_waves_to_a_tile_where_it_is_faster(tiles, B, D, O, G, F):
     assert _lib.lib().haste_ffi_bwd_features_tiles(B, D, F, O, G, 0) == tiles
 
 
+@pytest.mark.parametrize("joined,B,F,O,G", [
+    (1, 512, 128, 131073, 64), (1, 256, 256, 500000, 32), (1, 1024, 128, 3000000, 128),
+    (1, 16, 32, 4096, 32), (1, 300, 96, 3000, 64), (1, 512, 64, 670091, 64),
+    # measured slower: 42 -> 45 us, 91 -> 96, 86 -> 89, 352 -> 377
+    (0, 512, 128, 2000, 64), (0, 1, 32, 300001, 128), (0, 16, 96, 131073, 64),
+    (0, 1, 96, 510000, 32),
+    # no build
+    (0, 64, 256, 4096, 128),
+])
+def test_joined_update_and_logits_where_it_is_faster(joined, B, F, O, G):
+    f = _lib.lib().haste_ffi_forward_bwd_weights_joined
+    ld = (O + 63) // 64 * 64
+    assert f(64, ld, ld, B, F, O, G) == joined
+    assert f(66, ld, ld, B, F, O, G) == 0 and f(64, ld + 1, ld, B, F, O, G) == 0  # off 16 bytes
+
+
 def test_plans_of_alternating_layers_cost_no_tail_sums():
     """The bwd-features plan, made on every call, keeps its binomial tail sums: for
     the shapes of three layers in turn it takes about the time of one without any."""

@@ -3,6 +3,7 @@ haste_ffi_forward_bwd_weights_sgd_dx) against the calls it joins, bit for bit.""
 import pytest
 import torch
 
+from haste_amd import _lib
 from haste_amd.step import FFITrainStep
 
 pytestmark = pytest.mark.gpu
@@ -81,13 +82,15 @@ def test_rows_off_16_bytes_and_dY_in_the_logits(dev):
     assert torch.equal(a.logits, b.logits) and torch.equal(a.W, b.W) and torch.equal(a.dX, b.dX)
 
 
-def test_step_is_its_parts_with_streamed_dY(dev):
+@pytest.mark.parametrize("G,F", [(16, 32), (64, 64), (128, 128)])
+def test_step_is_its_parts_with_streamed_dY(dev, G, F):
     """dY just above the size from which the launch loads it without keeping it in the caches."""
-    B, D, O, G, F = 512, 300, 270001, 64, 64
+    B, D, O = 512, 300, 270001
     x, W, bias, idx, dY = case(dev, B, D, O, G, F)
     ld = (O + 7) // 8 * 8
     dY = dY[:, :ld].contiguous()
     assert (256 << 20) < dY.numel() * 2 < (272 << 20)
     a, b = both(dev, x, W, bias, idx, G, [(dY, ld)] * 2)
+    assert _lib.lib().haste_ffi_forward_bwd_weights_joined(dY.data_ptr(), ld, a.ldo, B, F, O, G) == 1
     assert torch.equal(a.logits, b.logits) and torch.equal(a.dX, b.dX)
     assert torch.equal(a.W, b.W) and torch.equal(a.bias, b.bias)

@@ -10,6 +10,7 @@ def bare(cls):
     """An instance without buffers on a device."""
     st = object.__new__(cls)
     st.grad_dtype, st.ldo, st.loss_buf = torch.float32, 64, torch.zeros(())
+    st._joins = {(64, 0): 1}
     st.logits_buf = torch.zeros(4, 64, dtype=torch.bfloat16)
     st.dY_buf = torch.zeros(4, 64, dtype=torch.bfloat16)
     return st
