@@ -283,21 +283,28 @@ inline BwdFPlan make_plan_for(int64_t B, int64_t D, int64_t F, int64_t O, int64_
 // Whether the staged plan p with two waves to a tile is faster than the other
 // builds' plan r.  Measured over some 2,500 shapes with B = 1 .. 1024, O = 3,000 ..
 // 670,091, D up to 4,500 and one to seven ranges (time of p / time of r, geometric
-// mean, extremes):
-//  - B <= 32: 0.63 (0.37 - 0.93);
-//  - fewer than 3/4 of r's workgroups (batches of 1024, whose units leave one
-//    slice): 1.07 (0.96 - 1.26) at G = 64 and 128, so r;
-//  - G = 64 and 128 otherwise: 0.74 (0.41 - 1.12) and 0.65 (0.29 - 1.15);
-//  - G = 32, whose products are one MFMA deep, so that what a group costs beside
-//    them counts: one range where r needs several, 0.70 (0.51 - 0.97; the fp32 layer
-//    at O = 131,073, F = 64, B = 256, D = 768: 104 -> 51 us), ranges that r covers in two
-//    tiles, 0.79 (0.55 - 1.03), or in three with the same batch tile, 0.71 (0.59 - 0.85);
-//  - G = 32 otherwise: 1.00 (0.52 - 1.48), above 1 for most of them, so r.
-inline bool half_pays(const BwdFPlan& p, const BwdFPlan& r, int64_t B, int64_t G) {
+// mean, extremes; "cold" with other data through the caches before each call):
+//  - B <= 32: 0.62 (0.37 - 0.97);
+//  - fewer workgroups than 3/4 of r's, or 7/8 at G = 32, which units of two or more
+//    batch tiles leave at large batches: 1.01 (0.57 - 1.48), cold 1.19, so r;
+//  - G = 64 and 128 otherwise: 0.74 (0.41 - 1.12) and 0.65 (0.29 - 1.15).
+// G = 32, whose products are one MFMA deep, so that what a group costs beside them counts:
+//  - one range where r needs several: 0.69 (0.36 - 0.97; the fp32 layer at O = 131,073,
+//    F = 64, B = 256, D = 768: 104 -> 51 us); one in both (D under 300): 1.12 (0.83 - 1.47),
+//    cold 0.90, so r;
+//  - several ranges whose tiles r holds in its full ring: 0.87 (0.78 - 0.98) from
+//    O = 262,144, cold 0.89; below 1.05 (0.95 - 1.16), cold 0.95, so r;
+//  - ranges that r covers in two tiles: 0.78 (0.55 - 1.03); in three, where p pads the
+//    batch less or has 64 rows too: 0.86 (0.52 - 1.23), cold 0.89; else 1.02 (0.71 - 1.24),
+//    cold 0.99, so r.
+inline bool half_pays(const BwdFPlan& p, const BwdFPlan& r, int64_t B, int64_t O, int64_t G) {
     if (B <= 32) return true;
-    if (4 * p.nbt * p.ndr * p.S < 3 * r.nbt * r.ndr * r.S) return false;
-    if (G > 32) return true;
-    return p.ndr == 1 ? r.ndr > 1 : r.RT == 2 || (r.RT == 3 && r.BT == p.BT);
+    const int64_t wp = p.nbt * p.ndr * p.S, wr = r.nbt * r.ndr * r.S;
+    if (G > 32) return 4 * wp >= 3 * wr;
+    if (8 * wp < 7 * wr) return false;
+    if (p.ndr == 1) return r.ndr > 1;
+    if (r.RT == ring_tiles(32)) return O >= 1 << 18;
+    return r.RT == 2 || p.BT == 64 || p.Bp < r.Bp;
 }
 
 // The plan of the build that haste_ffi_bwd_features_set_build selects (1 ring,
@@ -317,7 +324,7 @@ inline BwdFPlan make_plan(int64_t B, int64_t D, int64_t F, int64_t O, int64_t G)
     const bool fits = (p.gps + 8) * p.Tcap * 16 * G * 2 <= kMaxRsrcBytes;
     if (fits && (build == 3 || F >= 7 * 16 * p.ndr)) return p;
     const BwdFPlan r = make_plan_for(B, D, F, O, G, false);
-    return fits && p.tiles < kStagedTiles && half_pays(p, r, B, G) ? p : r;
+    return fits && p.tiles < kStagedTiles && half_pays(p, r, B, O, G) ? p : r;
 }
 
 // One 16-byte chunk (labels lc .. lc+7 of the group) of the W^T row described by

@@ -259,9 +259,10 @@ def test_half_cases_reach_every_build_with_two_waves_to_a_tile():
     # other builds split further
     (4, 512, 768, 670091, 64, 64), (4, 256, 768, 131073, 32, 64), (4, 16, 298, 3000, 32, 64),
     (4, 32, 4000, 20011, 128, 208), (4, 256, 1500, 300000, 64, 96),
+    (4, 64, 3524, 400001, 32, 256), (4, 96, 2130, 400001, 32, 144),
     # measured slower: 43 -> 64 us, 102 -> 132, 186 -> 275, 46 -> 58 (one slice)
     (0, 512, 201, 131073, 32, 64), (0, 256, 2090, 131073, 32, 176), (0, 400, 3321, 131073, 32, 144),
-    (0, 1024, 4061, 10007, 64, 192),
+    (0, 1024, 4061, 10007, 64, 192), (0, 256, 3524, 131073, 32, 256),
 ])
 def test_two_waves_to_a_tile_where_it_is_faster(tiles, B, D, O, G, F):
     assert _lib.lib().haste_ffi_bwd_features_tiles(B, D, F, O, G, 0) == tiles
