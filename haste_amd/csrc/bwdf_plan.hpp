@@ -57,7 +57,8 @@ __host__ __device__ constexpr int max_dc(int bt, int G, int rt) {
 // The staged build (bwdf_staged.hpp): kStagedTiles W^T tiles of a group's
 // range in its pipeline, dealt over its waves, and a ring of kStageBufs LDS
 // copies of the groups' dY tiles of bt rows x G labels beside the partial
-// (group i in buffer i % kStageBufs, staged kPlanWindow groups ahead).  Its
+// (group i in buffer i % kStageBufs, staged kPlanWindow groups ahead, or one more
+// where its operands are read early: StagedCfg::AHEAD).  Its
 // plan is made in windows of kPlanWindow groups (bwdf_plan_window_kernel) that
 // need no barrier between their partial updates; bit 31 of a group's meta
 // word 0 says it could not be laid out as part of its window.

@@ -7,8 +7,8 @@
 // CU), and an out-of-range buffer load costs as much as a real one.  So:
 //  - each group's dY tile [BT rows x G labels] is loaded once per workgroup,
 //    row-major (every thread one piece of PB bytes), and staged in LDS
-//    (a ring of six buffers, filled a plan window ahead; 16-byte chunks XOR-swizzled
-//    per row so that the operand reads of 16 rows hit distinct bank groups);
+//    (a ring of six buffers, filled AHEAD groups ahead, a plan window or one group more;
+//    16-byte chunks XOR-swizzled per row so that the operand reads of 16 rows hit distinct bank groups);
 //  - wave w owns W^T tile w of the range (16 positions): it loads that tile's
 //    operand fragments (chunk-major twt: one contiguous 1 KB per k-step) and
 //    the positions' partial-row offsets, reads the staged dY operands of all
@@ -449,7 +449,9 @@ __global__ __launch_bounds__(64 * W, 1) void bwdf_staged_kernel(
             // share in one wave's tile) the updates need none: it runs after
             // the iteration of a window's first group, and of a group the
             // plan could not lay out with its window; a tile staged
-            // kPlanWindow groups ahead is published by one of them in time.
+            // AHEAD groups ahead is published by one of them in time: as many
+            // iterations lie before its operands are read, less one where they
+            // are read an iteration early.
             const bool more = te - tb > TILES;  // uniform, rare
             if (K % kPlanWindow == 0 || (m[0] & kMetaUnpaired) || more) {
                 __builtin_amdgcn_s_waitcnt(wait_lgkmcnt(0));

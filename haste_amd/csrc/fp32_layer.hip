@@ -15,7 +15,7 @@ constexpr int kThreads = 256;
 // of 100: 28 us with a workgroup to a row, below the launch's 9 here).  in's rows start on
 // 4-byte boundaries only (its loads are unaligned 16-byte ones), out's on
 // 128-byte lines, so that the backward kernels take their aligned builds: torch's
-// cast left rows at in's stride, where the weight gradient took 36.5 us, now 29.8
+// cast left rows at in's stride, where the weight gradient took 36.5 us, here 29.8
 // (B = 256, O = 131,073, G = 32, F = 64), at the cost of torch's cast (28 us, 7.2 TB/s).
 __global__ __launch_bounds__(kThreads) void cast_rows_f16_kernel(const float* __restrict__ in,
                                                                  int64_t ldi,

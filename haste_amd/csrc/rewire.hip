@@ -318,10 +318,11 @@ __device__ __forceinline__ void load_pieces(u32x4 (&v)[NPT], rsrc_t rs, int tid)
 // otherwise they are computed here, without a gradient.  Bound by HBM: W is read
 // and written once (and by the Philox draws of RANDOM initial weights).  A given
 // score set took rewire_kernel's column stores before, 2 bytes per row of a
-// pruned slot: 41 us at 131,073 labels (G = 64, F = 128, RANDOM), 33 here.  A persistent grid: workgroup b takes groups b, b + gridDim.x,
-// ...; the next group's rows and indices are loaded into registers while the
-// current group is scored from LDS; a group with pruned slots goes back whole
-// with 16-byte stores; one atomic per workgroup adds its pruned count.  Pruned
+// pruned slot: 41 us at 131,073 labels (G = 64, F = 128, RANDOM), 33 here.
+// A persistent grid: workgroup b takes groups b, b + gridDim.x, ...; the next
+// group's rows and indices are loaded into registers while the current group
+// is scored from LDS; a group with pruned slots goes back whole with 16-byte
+// stores; one atomic per workgroup adds its pruned count.  Pruned
 // slots of idx get their RANDOM regrow index here, or -1 for the UNUSED pass
 // (rewire_regrow_kernel).  All global accesses go through buffer
 // resources with out-of-range offsets for the ones a lane skips, so that the
@@ -565,8 +566,8 @@ __global__ __launch_bounds__(kThreads) void rewire_regrow_kernel(int32_t* __rest
 // histograms the digit of the scores whose higher digits are settled; the next
 // launch's workgroups scan that histogram for the digit that holds rank k.  The
 // scores are read four times from the L2 (1 MB at 262,144 slots): the launches
-// bound it (five, 27 us at that size).  torch.kthvalue on 64-bit keys runs in one
-// workgroup: 1671 us there, and the whole rewire went from 1313 to 68 us.
+// bound it (five, 27 us at that size).  With torch.kthvalue on 64-bit keys, which runs
+// in one workgroup, the whole rewire took 1313 us there, and 68 with this.
 // Workspace (uint32): 3 histograms, the ties per chunk, then per pass the
 // settled digits and the rank left among the scores that share them.
 constexpr int kSelBins = 2048;
